@@ -27,7 +27,11 @@ GEMV_UNITS = [("kernels/gemv_inst.hip", f"gemv_inst_{w}_{x}",
               for w in range(4) for x in range(3)] + \
              [("kernels/gemv_inst.hip", f"gemv_inst_{w}_3",   # summed x (norm = 3): bf16 / fp8 weights
                [f"-DGEMV_WT={w}", "-DGEMV_XD=3", f"-DGEMV_PICK=gemv_pick_{w}_3"]) for w in (2, 3)]
-HIP_SOURCES = ["kernels/gemv.hip", "kernels/gemm.hip", "kernels/rowops.hip", "kernels/attn.hip",
+# the wide GEMM's instances: one unit per (weight type, x type, fused norm)
+WIDE_UNITS = [("kernels/gemm_wide_inst.hip", f"gemm_wide_inst_{w}_{x}_{n}",
+               [f"-DGW_WT={w}", f"-DGW_XT={x}", f"-DGW_NM={n}", f"-DGW_PICK=wide_pick_{w}_{x}_{n}"])
+              for w, x, n in ((2, 0, 0), (2, 0, 1), (2, 1, 0), (1, 0, 0), (1, 0, 1), (0, 1, 0))]
+HIP_SOURCES = ["kernels/gemv.hip", "kernels/gemm.hip", "kernels/gemm_wide.hip", "kernels/rowops.hip", "kernels/attn.hip",
                "kernels/mla.hip", "kernels/moe.hip", "kernels/step.hip", "kernels/step_m1.hip",
                "kernels/step_m2.hip", "kernels/step_m4.hip"]
 
@@ -81,12 +85,12 @@ def _build(OBJ: Path, LIB: Path, HIPFLAGS: list, verbose: bool, incremental: boo
         o = OBJ / (Path(s).stem + ".o")
         if not incremental or _stale(CSRC / s, o, hdr):
             jobs.append(["gcc", *CFLAGS, "-c", str(CSRC / s), "-o", str(o)])
-    units = [(s, Path(s).stem, []) for s in HIP_SOURCES] + GEMV_UNITS
+    units = [(s, Path(s).stem, []) for s in HIP_SOURCES] + GEMV_UNITS + WIDE_UNITS
     for s, stem, extra in units:
         o = OBJ / (stem + ".hip.o")
         if not incremental or _stale(CSRC / s, o, hdr):
             jobs.append([f"{ROCM}/bin/hipcc", *HIPFLAGS, *extra, "-c", str(CSRC / s), "-o", str(o)])
-    jobs.sort(key=lambda j: "gemv_inst" not in " ".join(j))    # the long units first
+    jobs.sort(key=lambda j: "_inst" not in " ".join(j))    # the long units first
     workers = max(1, min(len(jobs), int(os.environ.get("MAX_JOBS", "8"))))
     with cf.ThreadPoolExecutor(max_workers=workers) as ex:
         list(ex.map(_run, jobs))

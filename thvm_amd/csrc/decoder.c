@@ -209,6 +209,11 @@ static u32 tiled_copy(Decoder *d, u32 src, u32 n, u32 k, u32 wt, u32 lb) {
 
 static int op_add_raw(Decoder *d, const char *name, const char *prog, const u32 *args, u32 n);
 
+static u32 gemm_ws(Decoder *d) {
+  const u32 id = tens_find(d, "gemm.ws");
+  return id ? id : tens_new(d, "gemm.ws", THVM_DT_FP32, thvm_k_gemm_wide_ws_max());
+}
+
 static int op_add(Decoder *d, const char *name, const char *prog, const u32 *args, u32 n) {
   if (n >= 3 && d->rows > 4 && wtile_on() && strncmp(prog, "thvm-builtin:gemv ", 18) == 0 &&
       prog_u32(prog, "path", 0) != 1 && prog_u32(prog, "m", 0) > 4) {
@@ -218,14 +223,19 @@ static int op_add(Decoder *d, const char *name, const char *prog, const u32 *arg
                      ((wt == THVM_DT_FP16 && xt == THVM_DT_FP16) ||
                                      (wt == THVM_DT_BF16 && xt == THVM_DT_BF16) ||
                                      (wt == THVM_DT_FP8E4M3 && (xt == THVM_DT_BF16 || xt == THVM_DT_FP16)));
-    if (mfma && n <= 24 && strlen(prog) + 10 < 1024) {
+    if (mfma && n <= 24 && strlen(prog) + 16 < 1024) {
       const u32 tw = tiled_copy(d, args[2], prog_u32(prog, "n", 0), k, wt, 16 * hb_dt_size(wt));
       if (!tw) return -1;
       u32 a2[24];
       memcpy(a2, args, n * sizeof(u32));
       a2[2] = tw;
       char p2[1024];
-      snprintf(p2, sizeof p2, "%s tiled=1", prog);
+      /* above 16 rows: the wide GEMM's workspace (one per decoder: its ops run
+       * one after another), shapes it does not suit run as before */
+      const u32 ws = d->rows > 16 && n < 24 ? gemm_ws(d) : 0;
+      if (d->rows > 16 && n < 24 && !ws) return -1;
+      if (ws) a2[n++] = ws;
+      snprintf(p2, sizeof p2, "%s tiled=1%s", prog, ws ? " ws=1" : "");
       return op_add_raw(d, name, p2, a2, n);
     }
   }

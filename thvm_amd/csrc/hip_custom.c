@@ -202,7 +202,8 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
          spec_u32(&sp, "u", &a.tune_u, 0, 0) || spec_u32(&sp, "blocks", &a.tune_blocks, 0, 0) ||
          spec_u32(&sp, "path", &a.tune_path, 0, 0) || spec_u32(&sp, "spec", &a.spec, 0, 0) ||
          spec_u32(&sp, "tiled", &a.wtiled, 0, 0) || spec_u32(&sp, "clk", &a.clk_cap, 0, 0) ||
-         spec_u32(&sp, "xqs", &a.xqs, 0, a.K));
+         spec_u32(&sp, "xqs", &a.xqs, 0, a.K) || spec_u32(&sp, "ws", &a.wide, 0, 0) ||
+         spec_u32(&sp, "seq", &a.seq, 0, 0));
     {
       u32 ldy0 = a.epi == THVM_EPI_SWIGLU ? a.N / 2
                : (a.epi == THVM_EPI_QKV || a.epi == THVM_EPI_QKV_ROPE) ? a.n_heads * a.head_dim
@@ -233,13 +234,24 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
       a.rope_sin = (const float *)arg(&c, slot++, (u64)a.max_seq * (a.head_dim / 2) * 4);
     }
     if (qkv) {
-      u64 cb = (u64)(a.spec ? 1 : a.M) * a.n_kv_heads * a.max_seq * a.head_dim * ysz;
+      if (a.seq && (a.spec || !a.wide || a.M % a.seq)) {
+        hb_set_error("builtin gemv: seq=%u rows a sequence must divide m=%u, with ws=1 and without spec", a.seq, a.M);
+        return -1;
+      }
+      u64 cb = (u64)(a.spec ? 1 : a.seq ? a.M / a.seq : a.M) * a.n_kv_heads * a.max_seq * a.head_dim * ysz;
       a.len = (const int32_t *)arg(&c, slot++, 4);
       a.kcache = arg(&c, slot++, cb);
       a.vcache = arg(&c, slot++, cb);
     }
     /* clk=<blocks>: a phase-clock buffer after the others (blocks x 10 u64) */
     if (a.clk_cap) a.clk = (uint64_t *)arg(&c, slot++, (u64)a.clk_cap * 80);
+    /* ws=1: the workspace of the wide GEMM's K splits, last */
+    if (a.wide) {
+      const u64 need = thvm_k_gemm_wide_ws(&a);
+      a.ws = arg(&c, slot, need);
+      a.ws_bytes = a.ws ? hb_buf_size(ids[slot]) : 0;
+      slot++;
+    }
     if (c.bad) return -1;
     bytes = (u64)a.N * a.K * wsz + (a.scale ? (u64)a.N * 4 : 0) + (u64)a.M * a.K * (a.norm == 3 ? 16 : xsz) +
             (u64)a.M * ncols_out * ysz * (a.res ? 2 : 1);

@@ -79,6 +79,14 @@ typedef struct ThvmGemvArgs {
    * first clk_cap blocks */
   uint64_t *clk;
   uint32_t clk_cap;
+  /* the wide MFMA GEMM (gemm_wide.hip; taken when wide is set): workspace of
+   * its K splits, zero before the first launch (each launch leaves its
+   * counters zero); rows per sequence (seq > 0, the QKV epilogues): row m is
+   * position L-1 + m % seq of sequence m / seq.  splits and vec4 are the
+   * launcher's. */
+  uint32_t wide, seq, splits, vec4;
+  void *ws;
+  uint64_t ws_bytes;
 } ThvmGemvArgs;
 /* W [N, K] (row-major, element size es 1 or 2) -> the MFMA tile layout for
  * lanes reading lb bytes of a row per k step (lb 16 or 32, 0 = 16 es; a step
@@ -98,6 +106,13 @@ int thvm_k_tile_w(void *y, const void *w, uint32_t N, uint32_t K, uint32_t es, u
  * fused norm). */
 int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen);
 int thvm_k_gemm_mfma(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen);
+/* The same for many x rows (above 16; prompt chunks of hundreds): x shared by
+ * a block's waves, K split over blocks; _ws: bytes of workspace this shape
+ * needs, _ws_max: what any shape needs at the picked splits. */
+int thvm_k_gemm_wide(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen);
+int thvm_k_gemm_wide_use(const ThvmGemvArgs *a);   /* whether ws=1 takes it at this shape */
+uint64_t thvm_k_gemm_wide_ws(const ThvmGemvArgs *a);
+uint64_t thvm_k_gemm_wide_ws_max(void);
 
 /* Row norms over [M, K]: RMSNorm (y = rnd((x*inv)*w), inv=1/sqrt(ss/K+eps))
  * or LayerNorm (y = rnd((x-mu)*rsqrt(var+eps)*w + b)).  x may be f32/bf16/f16,

@@ -1,0 +1,139 @@
+// gemm_wide.hip -- launcher of the wide MFMA GEMM (gemm_wide_core.h): checks,
+// tile and split choice, launch.
+#include "gemm_wide_core.h"
+#include "launch.h"
+#include <stdio.h>
+
+typedef void (*wide_fn)(ThvmGemvArgs);
+// one picker per (weight type, x type, fused norm), each in its own unit
+#define WIDE_PICKERS(X) X(2, 0, 0) X(2, 0, 1) X(2, 1, 0) X(1, 0, 0) X(1, 0, 1) X(0, 1, 0)
+#define WIDE_DECL(w, x, n) wide_fn wide_pick_##w##_##x##_##n(int MT, int NT);
+WIDE_PICKERS(WIDE_DECL)
+#undef WIDE_DECL
+
+// Where this kernel takes over from k_gemm (16 < M <= 64; above it is the only
+// one).  k_gemm's x reads grow with M K N / (16 NT), this one pays a longer
+// chain per block (a barrier per 128 k, the split hand-off).  Measured on
+// gfx950, cold fp8 weights in a graph, k_gemm against this kernel, us:
+//   28672 x 4096  M 17 33.4 / 23.8   M 60 50.0 / 31.5      wide N
+//   14336 x 2048  M 17 10.6 /  8.0   M 60 16.3 / 11.2
+//   32000 x 1024  M 17 13.7 /  9.2   M 60 20.1 / 11.7
+//    4096 x 14336 M 17 17.8 / 14.5   M 60 33.6 / 19.2      long K
+//    2048 x 8192  M 17 10.4 /  9.1   M 60 18.4 / 12.2
+//    6144 x 4096  M 17 11.5 / 11.5   M 60 18.7 / 16.4      middling: by M
+//    4096 x 4096  M 17  7.5 /  8.2   M 60 11.9 / 10.5
+//    2048 x 4096  M 17  7.2 /  7.2   M 60 11.4 /  9.6
+//    6400 x 1600  M 17  6.4 /  7.0   M 60  9.3 /  9.5      small: k_gemm
+//    1600 x 1600  M 17  5.1 /  6.5   M 60  7.1 /  8.8
+extern "C" int thvm_k_gemm_wide_use(const ThvmGemvArgs *a) {
+  if (a->M <= 16) return 0;
+  return a->M > 64 || a->N >= 10240 || a->K >= 6144 || (a->M > 32 && (uint64_t)a->N * a->K >= (8u << 20));
+}
+
+// Tile and splits.  One block of 8 waves is resident per CU (more than 128
+// VGPRs), so the grid is planned in rounds of 256 blocks.
+//   * one tile of x rows (M <= 64; bound by the weight stream): 64 weight rows
+//     per block while that makes at most 256 blocks, else 128, and 256 for the
+//     widest N (an LM head runs many rounds anyway: 128256 x 4096 at M = 60,
+//     113 us with 128 rows, 102 with 256);
+//   * several (prompt chunks; bound by the MFMA and LDS pipes): the cheapest of
+//     64, 128, 256 rows by rounds x chunks x the measured time of a chunk
+//     (0.40, 0.56 and 1.04 us), e.g. at M = 299: 6144 x 4096 128 rows 22.4 us
+//     against 256 26.5, 4096 x 14336 256 rows in 3 splits 47.5 against 58;
+//   * splits fill the last round only (blocks * splits <= 256): a split costs
+//     its hand-off (~4 chunks) and a read of its tile (~1 chunk), and a block
+//     runs its chunks in fours.
+static void wide_plan(const ThvmGemvArgs *a, int *MT, int *NT, uint32_t *SP) {
+  *MT = a->M <= 32 ? 2 : 4;
+  const uint32_t mt = (a->M + 16u * *MT - 1) / (16u * *MT), g64 = (a->N + 63) / 64;
+  const uint32_t CH = (a->K / 64 + GW_KG - 1) / GW_KG;
+  static const float chunk[3] = {0.40f, 0.56f, 1.04f};
+  float best = 0.f;
+  *NT = 1;
+  *SP = 1;
+  for (int i = 0; i < 3; i++) {
+    const int nt = 1 << i;
+    if (a->tune_r ? (int)a->tune_r != nt : mt == 1 && nt != (g64 <= 256 ? 1 : g64 <= 512 ? 2 : 4)) continue;
+    const uint32_t blocks = (g64 + nt - 1) / nt * mt;
+    const uint32_t smax = a->tune_blocks ? a->tune_blocks : blocks >= 256 ? 1 : 256 / blocks < 8 ? 256 / blocks : 8;
+    for (uint32_t sp = a->tune_blocks ? smax : 1; sp <= smax && (sp == 1 || 4 * sp <= CH); sp++) {
+      const uint64_t per = ((CH + sp - 1) / sp + 3) / 4 * 4, rounds = ((uint64_t)blocks * sp + 255) / 256;
+      const float t = chunk[i] * (float)(rounds * per) + (sp > 1 ? 0.40f * (float)(4 + sp) : 0.f);
+      if (best == 0.f || t < best) { best = t; *NT = nt; *SP = sp; }
+    }
+  }
+}
+
+// bytes the splits of this call need
+extern "C" uint64_t thvm_k_gemm_wide_ws(const ThvmGemvArgs *a) {
+  int MT, NT;
+  uint32_t SP;
+  if (!thvm_k_gemm_wide_use(a)) return 0;
+  wide_plan(a, &MT, &NT, &SP);
+  if (SP <= 1) return 0;
+  const uint64_t tiles = (uint64_t)((a->N + 64u * NT - 1) / (64u * NT)) * ((a->M + 16u * MT - 1) / (16u * MT));
+  return GW_CTR_BYTES + tiles * SP * (GW_NWAVES * NT * MT * 1024ull + 16ull * MT * 4);
+}
+
+// splits are planned within 256 blocks, of at most 256 x 64 tiles
+extern "C" uint64_t thvm_k_gemm_wide_ws_max(void) {
+  return GW_CTR_BYTES + 256ull * (GW_NWAVES * 4 * 4 * 1024ull + 64 * 4);
+}
+
+extern "C" int thvm_k_gemm_wide(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen) {
+  if (a->norm && (a->norm != 1 || a->xdt != THVM_DT_BF16 || a->norm_w == nullptr)) {
+    snprintf(err, errlen, "gemm_wide: fuses RMSNorm with a gain over bf16 x only");
+    return -1;
+  }
+  if (a->tune_r && a->tune_r != 1 && a->tune_r != 2 && a->tune_r != 4) {
+    snprintf(err, errlen, "gemm_wide: r (64-row weight tiles per block) must be 1, 2 or 4");
+    return -1;
+  }
+  if (a->K % 64 || ((uint64_t)a->ldx * 2) % 16 || ((uintptr_t)a->x & 15) || ((uintptr_t)a->w & 15)) {
+    snprintf(err, errlen, "gemm_wide: K a multiple of 64, x rows and W 16-byte aligned");
+    return -1;
+  }
+  if (64ull * a->ldx * 2 >= (1ull << 31) || 64ull * a->K * (a->wdt == THVM_DT_FP8E4M3 ? 1 : 2) >= (1ull << 30)) {
+    snprintf(err, errlen, "gemm_wide: 64 rows of x or W exceed 1 GiB");
+    return -1;
+  }
+  int MT, NT;
+  uint32_t SP;
+  wide_plan(a, &MT, &NT, &SP);
+  ThvmGemvArgs k = *a;
+  k.splits = SP;
+  if (SP > 1 && (uint64_t)((a->N + 64u * NT - 1) / (64u * NT)) * ((a->M + 16u * MT - 1) / (16u * MT)) > GW_CTR_BYTES / 4) {
+    snprintf(err, errlen, "gemm_wide: %u splits of more than %u tiles", SP, GW_CTR_BYTES / 4);
+    return -1;
+  }
+  if (SP > 1 && (a->ws == nullptr || a->ws_bytes < thvm_k_gemm_wide_ws(a))) {
+    snprintf(err, errlen, "gemm_wide: %u splits need %llu bytes of workspace", SP,
+             (unsigned long long)thvm_k_gemm_wide_ws(a));
+    return -1;
+  }
+  const int xbf = a->xdt == THVM_DT_BF16, xf16 = a->xdt == THVM_DT_FP16;
+  wide_fn f = nullptr;
+  const int w = a->wdt == THVM_DT_FP8E4M3 ? GW_FP8 : a->wdt == THVM_DT_BF16 ? GW_BF16 : a->wdt == THVM_DT_FP16 ? GW_F16 : -1;
+  const int x = xbf ? GX_BF16 : xf16 ? GX_F16 : -1, nm = a->norm ? 1 : 0;
+  static_assert(GW_F16 == 0 && GW_BF16 == 1 && GW_FP8 == 2 && GX_BF16 == 0 && GX_F16 == 1, "picker numbering");
+#define WIDE_CASE(W, X, Q) if (w == W && x == X && nm == Q) f = wide_pick_##W##_##X##_##Q(MT, NT);
+  WIDE_PICKERS(WIDE_CASE)
+#undef WIDE_CASE
+  if (!f) { snprintf(err, errlen, "gemm_wide: no kernel for w=%u x=%u NT=%d", a->wdt, a->xdt, NT); return -1; }
+  // four rows per lane at a time where every row and buffer is aligned for it
+  const uintptr_t al = a->ydt == THVM_DT_FP32 ? 15 : 7;
+  const bool qkv = a->epi == THVM_EPI_QKV || a->epi == THVM_EPI_QKV_ROPE;
+  k.vec4 = a->N % 4 == 0 && a->ldy % 4 == 0 && !((uintptr_t)a->y & al) && !((uintptr_t)a->res & al) &&
+           !((uintptr_t)a->bias & al) && !((uintptr_t)a->scale & 15) &&
+           (!qkv || (a->head_dim % 4 == 0 && !((uintptr_t)a->kcache & al) && !((uintptr_t)a->vcache & al) &&
+                     !((uintptr_t)a->rope_cos & 7) && !((uintptr_t)a->rope_sin & 7)));
+  const uint32_t mt = (a->M + 16u * MT - 1) / (16u * MT), nt = (a->N + 64u * NT - 1) / (64u * NT);
+  const uint64_t total = (uint64_t)mt * nt * SP, grid = (total + 7) / 8 * 8;
+  if (grid > 0x7fffffffull) { snprintf(err, errlen, "gemm_wide: grid too large"); return -1; }
+  const uint32_t xlds = 2u * 16u * MT * GW_XROW, elds = (uint32_t)GW_NWAVES * NT * MT * 1024u;
+  const uint32_t lds = xlds > elds ? xlds : elds;
+  thvm_launch(true, true, f, dim3((uint32_t)grid), dim3(GW_THREADS), lds, s, k);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { snprintf(err, errlen, "gemm_wide launch: %s", hipGetErrorString(e)); return -1; }
+  return 0;
+}

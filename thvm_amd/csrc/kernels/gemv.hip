@@ -54,8 +54,8 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
     snprintf(err, errlen, "gemv: unsupported dtypes w=%u x=%u y=%u", a->wdt, a->xdt, a->ydt);
     return -1;
   }
-  if (a->M < 1 || a->M > 64 || a->N == 0 || a->K == 0) {
-    snprintf(err, errlen, "gemv: M=%u N=%u K=%u out of range (M in 1..64)", a->M, a->N, a->K);
+  if (a->M < 1 || (a->M > 64 && !a->wide) || a->M > 65536 || a->N == 0 || a->K == 0) {
+    snprintf(err, errlen, "gemv: M=%u N=%u K=%u out of range (M in 1..64, 65536 with ws=1)", a->M, a->N, a->K);
     return -1;
   }
   if (((uint64_t)a->K * wsz) % 16 != 0) {
@@ -142,6 +142,13 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
         ((a->wdt == THVM_DT_FP16 && a->xdt == THVM_DT_FP16) || (a->wdt == THVM_DT_BF16 && a->xdt == THVM_DT_BF16) ||
          (a->wdt == THVM_DT_FP8E4M3 && (a->xdt == THVM_DT_BF16 || a->xdt == THVM_DT_FP16)));
     const bool mfma = a->tune_path == 2 || (a->tune_path == 0 && mfma_types && (a->M > 4 || xlds > 160 * 1024));
+    if (a->wide && a->tune_path != 1 && thvm_k_gemm_wide_use(a)) {
+      if (!mfma_types) {
+        snprintf(err, errlen, "gemv: ws=1 takes 16-bit x, fp8 or the x type's weights, K %% 64 == 0 and no norm but RMSNorm over bf16");
+        return -1;
+      }
+      return thvm_k_gemm_wide(a, s, err, errlen);
+    }
     if (mfma) return thvm_k_gemm_mfma(a, s, err, errlen);
     if (a->wtiled) {
       snprintf(err, errlen, "gemv: tiled weights run on the MFMA path only (M > 4, 16-bit x, K %% 64 == 0)");
