@@ -31,7 +31,7 @@ GEMV_UNITS = [("kernels/gemv_inst.hip", f"gemv_inst_{w}_{x}",
 WIDE_UNITS = [("kernels/gemm_wide_inst.hip", f"gemm_wide_inst_{w}_{x}_{n}",
                [f"-DGW_WT={w}", f"-DGW_XT={x}", f"-DGW_NM={n}", f"-DGW_PICK=wide_pick_{w}_{x}_{n}"])
               for w, x, n in ((2, 0, 0), (2, 0, 1), (2, 1, 0), (1, 0, 0), (1, 0, 1), (0, 1, 0))]
-HIP_SOURCES = ["kernels/gemv.hip", "kernels/gemm.hip", "kernels/gemm_wide.hip", "kernels/rowops.hip", "kernels/attn.hip",
+HIP_SOURCES = ["kernels/gemv.hip", "kernels/gemm.hip", "kernels/gemm_wide.hip", "kernels/rowops.hip", "kernels/attn.hip", "kernels/attn_prompt.hip",
                "kernels/mla.hip", "kernels/moe.hip", "kernels/step.hip", "kernels/step_m1.hip",
                "kernels/step_m2.hip", "kernels/step_m4.hip"]
 

@@ -1228,6 +1228,158 @@ THVM_API int thvm_hip_decoder_set_state(uint32_t h, const int32_t *tokens, uint3
   return 0;
 }
 
+/* ---- prompt ingestion ----------------------------------------------------
+ * generate() reads a prompt in chunks of up to PROMPT_ROWS rows (B sequences x
+ * T positions) through the layers -- one pass over the weights per chunk, on
+ * the wide GEMM and the causal chunk attention -- where the captured step
+ * would read them once per position.  Projections and norms round where the
+ * step rounds.  Measured on gfx950, four Llama-8B-shape fp8 layers and a
+ * 128256 head, a step at a time against chunks: 300 ids 109 / 1.39 ms, 24 ids
+ * 8.9 / 0.60, 2 ids 0.77 / 0.50; four layers of width 1024, 2 ids 0.36 / 0.27.
+ * So every prompt of two ids or more goes this way, except for models the
+ * chunk kernels do not take (f32 activations, weights of another 16-bit type,
+ * MLA, the persistent step).  512 rows: the projections' time per row is flat
+ * from there on (4096 x 28672: 0.33 us at 299 rows, 0.27 at 512). */
+#define PROMPT_ROWS 512
+
+static int prompt_can(const Decoder *d) {
+  const ThvmDecodeConfig *c = &d->c;
+  if ((c->arch != THVM_ARCH_LLAMA && c->arch != THVM_ARCH_GPT2) || c->step_mode) return 0;
+  if (c->adtype != THVM_DT_BF16 && c->adtype != THVM_DT_FP16) return 0;
+  if (c->wdtype != c->adtype && c->wdtype != THVM_DT_FP8E4M3) return 0;
+  return c->dim % 64 == 0 && (c->n_heads * c->head_dim) % 64 == 0 && c->ffn % 64 == 0;
+}
+
+/* layer l's tensor; tiled: its tiled copy where there is one */
+static u32 ltens(Decoder *d, u32 l, const char *name, const char *suffix, int *tiled) {
+  char nm[48];
+  snprintf(nm, sizeof nm, "l%u.%s%s", l, name, suffix);
+  if (!tiled) return tens_find(d, nm);
+  char tn[56];
+  snprintf(tn, sizeof tn, "%s.tiled", nm);
+  const u32 t = tens_find(d, tn);
+  *tiled = t != 0;
+  return t ? t : tens_find(d, nm);
+}
+
+/* y = epi(x W^T) for `rows` rows; extra: the spec's further keys */
+static int prompt_gemm(Decoder *d, u32 l, const char *w, u32 rows, u32 n, u32 k, u32 epi, const char *extra,
+                       u32 y, u32 x, const u32 *more, u32 nmore) {
+  const ThvmDecodeConfig *c = &d->c;
+  char p[400];
+  int tiled = 0;
+  u32 a[12], na = 0;
+  a[na++] = y;
+  a[na++] = x;
+  a[na++] = ltens(d, l, w, "", &tiled);
+  if (c->wdtype == THVM_DT_FP8E4M3) a[na++] = ltens(d, l, w, ".scale", NULL);
+  if (c->arch == THVM_ARCH_GPT2) a[na++] = ltens(d, l, w, ".b", NULL);
+  for (u32 i = 0; i < nmore; i++) a[na++] = more[i];
+  a[na++] = tens_find(d, "gemm.ws");
+  snprintf(p, sizeof p, "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=%u bias=%d tiled=%d ws=1%s", rows, n, k,
+           c->wdtype, c->adtype, c->adtype, epi, c->arch == THVM_ARCH_GPT2, tiled, extra);
+  return run_now(p, a, na);
+}
+
+static int prompt_norm(Decoder *d, u32 rows, u32 xn, u32 x, u32 g, u32 b) {
+  const ThvmDecodeConfig *c = &d->c;
+  char p[200];
+  const u32 a[4] = {xn, x, g, b};
+  snprintf(p, sizeof p, "thvm-builtin:norm m=%u k=%u xt=%u yt=%u eps=%a ln=%d bias=%d", rows, c->dim, c->adtype,
+           c->adtype, c->eps, b != 0, b != 0);
+  return run_now(p, a, b ? 4 : 3);
+}
+
+/* the layers over T positions of each sequence from position len - 1 (both in
+ * place already): p.tok -> p.x and the caches */
+static int prompt_layers(Decoder *d, u32 T) {
+  const ThvmDecodeConfig *c = &d->c;
+  const u32 B = c->batch, rows = B * T, D = c->dim, H = c->n_heads, Hkv = c->n_kv_heads, hd = c->head_dim, F = c->ffn;
+  const int gpt = c->arch == THVM_ARCH_GPT2;
+  const u32 x = tens_find(d, "p.x"), xn = tens_find(d, "p.xn"), q = tens_find(d, "p.q"), att = tens_find(d, "p.att"),
+            h = tens_find(d, "p.h"), L = tens_find(d, "len");
+  char p[320], ex[160];
+  snprintf(p, sizeof p, "thvm-builtin:embed b=%u d=%u v=%u et=%u xt=%u pos=%d maxseq=%u seq=%u", rows, D, c->vocab,
+           c->adtype, c->adtype, gpt, c->max_seq, T);
+  const u32 ea[5] = {x, tens_find(d, gpt ? "wte" : "emb"), tens_find(d, "p.tok"), tens_find(d, "wpe"), L};
+  if (run_now(p, ea, gpt ? 5 : 3)) return -1;
+  for (u32 l = 0; l < c->n_layers; l++) {
+    const u32 kc = ltens(d, l, "kcache", "", NULL), vc = ltens(d, l, "vcache", "", NULL);
+    if (prompt_norm(d, rows, xn, x, ltens(d, l, gpt ? "ln1.g" : "g_attn", "", NULL), gpt ? ltens(d, l, "ln1.b", "", NULL) : 0))
+      return -1;
+    snprintf(ex, sizeof ex, " h=%u hkv=%u hd=%u maxseq=%u seq=%u", H, Hkv, hd, c->max_seq, T);
+    const u32 qa[5] = {tens_find(d, "rope.cos"), tens_find(d, "rope.sin"), L, kc, vc};
+    if (prompt_gemm(d, l, gpt ? "c_attn" : "wqkv", rows, (H + 2 * Hkv) * hd, D, gpt ? THVM_EPI_QKV : THVM_EPI_QKV_ROPE,
+                    ex, q, xn, gpt ? qa + 2 : qa, gpt ? 3 : 5))
+      return -1;
+    snprintf(p, sizeof p, "thvm-builtin:attn_prompt b=%u t=%u h=%u hkv=%u hd=%u maxseq=%u dt=%u scale=%a", B, T, H, Hkv,
+             hd, c->max_seq, c->adtype, (float)(1.0 / sqrt((double)hd)));
+    const u32 aa[5] = {att, q, kc, vc, L};
+    if (run_now(p, aa, 5)) return -1;
+    if (prompt_gemm(d, l, gpt ? "c_proj" : "wo", rows, D, H * hd, THVM_EPI_RESID, "", x, att, &x, 1)) return -1;
+    if (prompt_norm(d, rows, xn, x, ltens(d, l, gpt ? "ln2.g" : "g_ffn", "", NULL), gpt ? ltens(d, l, "ln2.b", "", NULL) : 0))
+      return -1;
+    if (prompt_gemm(d, l, gpt ? "c_fc" : "wgu", rows, gpt ? F : 2 * F, D, gpt ? THVM_EPI_GELU : THVM_EPI_SWIGLU, "", h, xn,
+                    NULL, 0) ||
+        prompt_gemm(d, l, gpt ? "mlp_proj" : "wd", rows, D, F, THVM_EPI_RESID, "", x, h, &x, 1))
+      return -1;
+  }
+  return 0;
+}
+
+/* Consume prompts [batch][ld], positions [0, n), leaving every buffer a step
+ * reads as n steps would; with tail, the logits and the next token of the last
+ * position too.  1 done, 0 not for this model or length, -1 failure. */
+int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 ld, u32 n, int tail) {
+  Decoder *d = dec_get(hdl);
+  if (!d) return -1;
+  const ThvmDecodeConfig *c = &d->c;
+  const u32 B = c->batch, D = c->dim, as = hb_dt_size(c->adtype);
+  if (n < 2 || !prompt_can(d) || thvm_hip_jit_is_capturing()) return 0;
+  for (u32 i = 0; i < n; i++)
+    for (u32 b = 0; b < B; b++) {
+      const int32_t t = prompts[(u64)b * ld + i];
+      if (t < 0 || (u32)t >= c->vocab) {
+        hb_set_error("decoder_generate: token %d of row %u outside [0, %u)", t, b, c->vocab);
+        return -1;
+      }
+    }
+  if (!tens_find(d, "p.x")) {            /* the chunk's workspace, kept with the decoder */
+    const u64 R = PROMPT_ROWS;
+    const u32 hq = c->n_heads * c->head_dim;
+    if (!gemm_ws(d) || !tens_new(d, "p.tok", THVM_DT_INT32, R * 4) || !tens_new(d, "p.xn", c->adtype, R * D * as) ||
+        !tens_new(d, "p.q", c->adtype, R * hq * as) || !tens_new(d, "p.att", c->adtype, R * hq * as) ||
+        !tens_new(d, "p.h", c->adtype, R * c->ffn * as) || !tens_new(d, "p.x", c->adtype, R * D * as))
+      return -1;
+  }
+  int32_t *tok = (int32_t *)malloc(PROMPT_ROWS * sizeof *tok);
+  if (!tok) { hb_set_error("decoder_generate: out of host memory"); return -1; }
+  int rc = 0;
+  u32 T = 0;
+  for (u32 p0 = 0; p0 < n && !rc; p0 += T) {
+    T = n - p0 < PROMPT_ROWS / B ? n - p0 : PROMPT_ROWS / B;
+    const int32_t L = (int32_t)p0 + 1;
+    for (u32 b = 0; b < B; b++) memcpy(tok + (u64)b * T, prompts + (u64)b * ld + p0, (u64)T * 4);
+    rc = thvm_hip_buf_write(tens_find(d, "p.tok"), tok, (u64)B * T * 4) ||
+         thvm_hip_buf_write(tens_find(d, "len"), &L, 4) || prompt_layers(d, T);
+  }
+  for (u32 b = 0; b < B && !rc; b++) {
+    rc = thvm_hip_buf_write_at(tens_find(d, "hist"), (u64)b * (c->max_seq + 1) * 4, prompts + (u64)b * ld, (u64)n * 4);
+    tok[b] = prompts[(u64)b * ld + n - 1];
+  }
+  if (!rc) rc = thvm_hip_decoder_set_state(hdl, tok, n - 1);
+  free(tok);
+  if (rc) return -1;
+  /* the last position's residual rows, where the step leaves them */
+  hipError_t e = hipMemcpy2DAsync(hb_buf_ptr(act(d, "x")), (u64)D * as,
+                                  (const char *)hb_buf_ptr(tens_find(d, "p.x")) + (u64)(T - 1) * D * as,
+                                  (u64)T * D * as, (u64)D * as, B, hipMemcpyDeviceToDevice, HB_STREAM);
+  if (e != hipSuccess) { hb_set_error("decoder_generate: %s", hipGetErrorString(e)); return -1; }
+  for (u32 i = 0; i < d->n_ops && tail; i++)
+    if (d->ops[i].tag == -2 && run_now(d->ops[i].prog, d->ops[i].args, d->ops[i].n_args)) return -1;
+  return 1;
+}
+
 THVM_API int thvm_hip_decoder_prefill_synthetic(uint32_t h, uint32_t ctx, uint64_t seed) {
   Decoder *d = dec_get(h);
   if (!d) return -1;

@@ -314,6 +314,27 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
     if (check_only) return 0;
     if (prof) hb_kprof_begin(K, &e0, &e1);
     rc = thvm_k_attn_decode(&a, HB_STREAM, err, sizeof err);
+  } else if (strcmp(K, "attn_prompt") == 0) {   /* out, q, kcache, vcache, len */
+    ThvmAttnArgs a;
+    memset(&a, 0, sizeof a);
+    NEED(spec_u32(&sp, "b", &a.B, 1, 0) || spec_u32(&sp, "t", &a.T, 1, 0) || spec_u32(&sp, "h", &a.H, 1, 0) ||
+         spec_u32(&sp, "hkv", &a.Hkv, 1, 0) || spec_u32(&sp, "hd", &a.hd, 1, 0) ||
+         spec_u32(&sp, "maxseq", &a.max_seq, 1, 0) || spec_u32(&sp, "dt", &a.cdt, 0, THVM_DT_BF16) ||
+         spec_f32(&sp, "scale", &a.scale, 1, 0));
+    a.qdt = a.odt = a.cdt;
+    if (!is_act(a.cdt)) { hb_set_error("builtin attn_prompt: bad dtype"); return -1; }
+    const u64 qb = (u64)a.B * a.T * a.H * a.hd * hb_dt_size(a.cdt);
+    const u64 cb = (u64)a.B * a.Hkv * a.max_seq * a.hd * hb_dt_size(a.cdt);
+    a.out = arg(&c, 0, qb);
+    a.q = arg(&c, 1, qb);
+    a.kcache = arg(&c, 2, cb);
+    a.vcache = arg(&c, 3, cb);
+    a.len = (const int32_t *)arg(&c, 4, 4);
+    if (c.bad) return -1;
+    bytes = 0;                       /* live-length dependent */
+    if (check_only) return 0;
+    if (prof) hb_kprof_begin(K, &e0, &e1);
+    rc = thvm_k_attn_prompt(&a, HB_STREAM, err, sizeof err);
   } else if (strcmp(K, "mla_prep") == 0 || strcmp(K, "mla_attn") == 0) {
     ThvmMlaArgs a;
     memset(&a, 0, sizeof a);
@@ -467,7 +488,7 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
     NEED(spec_u32(&sp, "b", &a.B, 1, 0) || spec_u32(&sp, "d", &a.D, 1, 0) ||
          spec_u32(&sp, "v", &a.V, 1, 0) || spec_u32(&sp, "et", &a.edt, 0, THVM_DT_BF16) ||
          spec_u32(&sp, "xt", &a.xdt, 0, THVM_DT_BF16) || spec_u32(&sp, "pos", &pos, 0, 0) ||
-         spec_u32(&sp, "maxseq", &a.max_seq, 0, 0));
+         spec_u32(&sp, "maxseq", &a.max_seq, 0, 0) || spec_u32(&sp, "seq", &a.seq, 0, 0));
     if (!is_act(a.edt) || !is_act(a.xdt)) { hb_set_error("builtin embed: bad dtypes"); return -1; }
     a.x = arg(&c, 0, (u64)a.B * a.D * hb_dt_size(a.xdt));
     a.emb = arg(&c, 1, (u64)a.V * a.D * hb_dt_size(a.edt));

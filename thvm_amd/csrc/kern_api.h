@@ -158,6 +158,7 @@ typedef struct ThvmAttnArgs {
                             * reads cache row 0 over L+b rows (causal)     */
   uint64_t *clk;           /* phase clock (measurement only; NULL = off)   */
   uint32_t clk_cap;        /* blocks recorded per launch (split, then merge) */
+  uint32_t T;              /* thvm_k_attn_prompt: positions per sequence     */
   uint32_t mf;             /* the split on MFMA (16-bit caches, hd 64 / 128,
                             * G <= 8, two launches): 0 picked from the shape
                             * (batched decode), 1 on, 2 off                 */
@@ -290,12 +291,19 @@ uint64_t thvm_k_moe_part_bytes(uint32_t B, uint32_t K, uint32_t D);
 int thvm_k_moe_gateup(const ThvmMoeArgs *a, hipStream_t s, char *err, int errlen);
 int thvm_k_moe_down(const ThvmMoeArgs *a, hipStream_t s, char *err, int errlen);
 
-/* Embedding gather: x[b][i] = emb[tok[b]][i] (+ pos[L-1][i] when pos != NULL),
- * tok int32 [B]; out of range ids read a zero row. */
+/* Causal attention of a prompt chunk: q and out [B][T][H][hd], position t of
+ * sequence b over its cache rows [0, L + t), which hold the chunk's own rows
+ * already; 16-bit types, hd 64 or 128.  Uses out, q, kcache, vcache, len, B,
+ * H, Hkv, hd, max_seq, qdt, cdt, odt, scale and T. */
+int thvm_k_attn_prompt(const ThvmAttnArgs *a, hipStream_t s, char *err, int errlen);
+
+/* Embedding gather: x[b][i] = emb[tok[b]][i] (+ pos[L-1][i] when pos != NULL;
+ * with seq > 0 pos[L-1 + b % seq][i]: seq positions of each sequence), tok
+ * int32 [B]; out of range ids read a zero row. */
 typedef struct ThvmEmbedArgs {
   void *x; const void *emb; const void *pos_emb; const int32_t *tok;
   const int32_t *len;
-  uint32_t B, D, V, max_seq, edt, xdt;
+  uint32_t B, D, V, max_seq, edt, xdt, seq;
 } ThvmEmbedArgs;
 int thvm_k_embed(const ThvmEmbedArgs *a, hipStream_t s, char *err, int errlen);
 

@@ -26,6 +26,7 @@ WIDE_PICKERS(WIDE_DECL)
 //    6400 x 1600  M 17  6.4 /  7.0   M 60  9.3 /  9.5      small: k_gemm
 //    1600 x 1600  M 17  5.1 /  6.5   M 60  7.1 /  8.8
 extern "C" int thvm_k_gemm_wide_use(const ThvmGemvArgs *a) {
+  if (a->seq) return 1;
   if (a->M <= 16) return 0;
   return a->M > 64 || a->N >= 10240 || a->K >= 6144 || (a->M > 32 && (uint64_t)a->N * a->K >= (8u << 20));
 }
@@ -127,6 +128,10 @@ extern "C" int thvm_k_gemm_wide(const ThvmGemvArgs *a, hipStream_t s, char *err,
            !((uintptr_t)a->bias & al) && !((uintptr_t)a->scale & 15) &&
            (!qkv || (a->head_dim % 4 == 0 && !((uintptr_t)a->kcache & al) && !((uintptr_t)a->vcache & al) &&
                      !((uintptr_t)a->rope_cos & 7) && !((uintptr_t)a->rope_sin & 7)));
+  if (a->seq && !k.vec4) {
+    snprintf(err, errlen, "gemm_wide: seq needs aligned rows of four (the scalar epilogue has one position per row)");
+    return -1;
+  }
   const uint32_t mt = (a->M + 16u * MT - 1) / (16u * MT), nt = (a->N + 64u * NT - 1) / (64u * NT);
   const uint64_t total = (uint64_t)mt * nt * SP, grid = (total + 7) / 8 * 8;
   if (grid > 0x7fffffffull) { snprintf(err, errlen, "gemm_wide: grid too large"); return -1; }

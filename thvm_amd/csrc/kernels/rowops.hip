@@ -304,7 +304,7 @@ __global__ void k_embed(ThvmEmbedArgs a) {
   float v = 0.0f;
   if (t >= 0 && (uint32_t)t < a.V) v = ld_a(a.emb, (uint64_t)t * a.D + i, a.edt);
   if (a.pos_emb) {
-    const int32_t p = a.len[0] - 1;
+    const int32_t p = a.len[0] - 1 + (a.seq ? (int32_t)(b % a.seq) : 0);
     if (p >= 0 && (uint32_t)p < a.max_seq) v = v + ld_a(a.pos_emb, (uint64_t)p * a.D + i, a.edt);
   }
   st_a(a.x, (uint64_t)b * a.D + i, a.xdt, v);

@@ -2,8 +2,8 @@
  *
  * Reference counterpart: the serve mode of bench/dsv2_decode_bench.c
  * (:2749-2897): weights and the captured step stay resident, a prompt is
- * consumed one position at a time by replaying the step with the prompt
- * token written into the device token buffer (:2769-2779), then the step
+ * consumed (there one position at a time, :2769-2779; here in chunks through
+ * the layers, hb_decoder_prompt, where the model allows), then the step
  * replays with the device-resident token, and generation stops at the eos
  * id (not emitted) or the per-request cap.  The line protocol is the
  * reference's: "ready" once, then per request line "id,id,...[|max_new]"
@@ -45,8 +45,11 @@ static int gen_step(uint32_t h) {
  * the one-row step finishes the request. */
 static int generate_spec(uint32_t h, const int32_t *prompt, uint32_t np, uint32_t max_new,
                          int32_t eos, int32_t *out, uint32_t *n_out, u32 S, u32 max_seq) {
-  int rc = 0;
-  for (u32 i = 0; i + 1 < np && !rc; i++) rc = thvm_hip_decoder_set_state(h, &prompt[i], i) || gen_step(h);
+  int rc = hb_decoder_prompt(h, prompt, np, np - 1, 0);
+  if (rc < 0) return -1;
+  const u32 i0 = rc ? np - 1 : 0;
+  rc = 0;
+  for (u32 i = i0; i + 1 < np && !rc; i++) rc = thvm_hip_decoder_set_state(h, &prompt[i], i) || gen_step(h);
   if (!rc) rc = thvm_hip_decoder_set_state(h, &prompt[np - 1], np - 1);
   int32_t *hist = (int32_t *)malloc((u64)(max_seq + 1) * 4);
   if (!hist) { hb_set_error("decoder_generate: out of host memory"); return -1; }
@@ -104,9 +107,12 @@ THVM_API int thvm_hip_decoder_generate(uint32_t h, const int32_t *prompts, uint3
   int32_t *tok = (int32_t *)malloc((u64)B * 4);
   int32_t *hist = (int32_t *)malloc((u64)B * (S + 1) * 4);
   if (!tok || !hist) { free(tok); free(hist); hb_set_error("decoder_generate: out of host memory"); return -1; }
-  int rc = 0;
-  /* prefill: position i consumes prompt id i (reference serve_prefill) */
-  for (u32 i = 0; i < n_prompt && !rc; i++) {
+  /* prefill: position i consumes prompt id i (reference serve_prefill), in
+   * chunks where the model and the length allow, else a step per position */
+  int rc = hb_decoder_prompt(h, prompts, n_prompt, n_prompt, 1);
+  const u32 i0 = rc > 0 ? n_prompt : 0;
+  if (rc > 0) rc = 0;
+  for (u32 i = i0; i < n_prompt && !rc; i++) {
     for (u32 b = 0; b < B; b++) tok[b] = prompts[(u64)b * n_prompt + i];
     rc = thvm_hip_decoder_set_state(h, tok, i) || gen_step(h);
   }
@@ -128,7 +134,8 @@ THVM_API int thvm_hip_decoder_generate(uint32_t h, const int32_t *prompts, uint3
     }
     if (done_rows == B || have == max_new) break;
     const u32 burst = max_new - have < 8 ? max_new - have : 8;
-    if (thvm_hip_decoder_replay(h, burst)) { rc = -1; break; }
+    const u32 first = hb_decoder_slot(h) ? 0 : 1;        /* the capture runs a step */
+    if ((first && gen_step(h)) || (burst > first && thvm_hip_decoder_replay(h, burst - first))) { rc = -1; break; }
     have += burst;
   }
   free(done);
