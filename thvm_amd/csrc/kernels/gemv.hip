@@ -170,18 +170,19 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
     }
   }
   // two rows per wave where a row fills at most half a batch of chunks (half
-  // the lanes would idle) over many rows per wave: measured on gfx950 at the
-  // C5 LM head (102400 x 2048 fp8), 53.5 -> 38.9 us.  A row's lanes and chunk
-  // order are unchanged, so the sums are bit-identical.  (One-shot GEMVs of
-  // the same rows measured no gain.)
-  if (!a->tune_r && R == 1 && a->N % 2 == 0 && a->N >= 32768 && a->M <= 4 &&
-      (uint64_t)a->K * wsz / 16 <= 128) {
+  // the lanes would idle) and one row per wave would take more than one block
+  // per CU, each staging x: measured on gfx950, 102400 x 2048 fp8 (the C5 LM
+  // head) 53.5 -> 38.9 us, 3648 x 2048 with a fused norm 5.9 -> 5.5 us at M = 1
+  // and 9.9 -> 9.1 at 4; 2048 x 2048 (256 blocks) 3.9 us stays.  A row's lanes
+  // and chunk order are unchanged, so the sums are bit-identical.
+  if (!a->tune_r && R == 1 && a->N % 2 == 0 && a->N > 2048 && a->M <= 4 && (uint64_t)a->K * wsz / 16 <= 128) {
     R = 2;
   }
-  // four x rows over long weight rows (>= 768 chunks): two rows per wave share
-  // each x read from LDS, which binds at M = 4 (measured on gfx950 at the C4
-  // down shape, 14336-wide fp8 rows: 24.7 -> 22.6 us); bit-identical sums
-  if (!a->tune_r && R == 1 && Mk == 4 && a->N % 2 == 0 && (uint64_t)a->K * wsz / 16 >= 768) R = 2;
+  // three or four x rows over long weight rows (>= 768 chunks): two rows per
+  // wave share each x read from LDS (measured on gfx950 at the C4 down shape,
+  // 14336-wide fp8 rows: M = 3 21.2 -> 17.1 us, M = 4 23.3 -> 18.8; at M = 2 one
+  // row is faster, 14.0 against 15.8); bit-identical sums
+  if (!a->tune_r && R == 1 && Mk >= 3 && a->N % 2 == 0 && (uint64_t)a->K * wsz / 16 >= 768) R = 2;
   if (a->tune_r) {
     if (a->tune_r != 1 && a->tune_r != 2) { snprintf(err, errlen, "gemv: r must be 1 or 2"); return -1; }
     if ((pairs && a->tune_r == 1) || a->N % a->tune_r) { snprintf(err, errlen, "gemv: r=%u does not tile N/epilogue", a->tune_r); return -1; }
@@ -227,6 +228,7 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
       (Gr + 7) / 8 > 256 && (Gr + 15) / 16 <= 256) {
     waves = (Gr + 255) / 256;
   }
+  if (Mk > 1 && waves > 8) waves = 8;   // the instances' block limit; the sums do not depend on it
   if (xsum && a->K > 2u * GEMV_SQ * 64u * waves) {   // the staging's element pairs per thread
     snprintf(err, errlen, "gemv: norm=3 needs K <= %u at %u waves per block", 2u * GEMV_SQ * 64u * waves, waves);
     return -1;

@@ -160,6 +160,30 @@ __device__ __forceinline__ float block_sum_g(float v, float *red, int nwaves) {
   return t;
 }
 
+// the same for M rows at once: one pair of barriers, each row's sum with
+// block_sum_g's additions (red: M x GEMV_MAX_WAVES)
+template <int M>
+__device__ __forceinline__ void block_sum_m(float (&v)[M], float *red, int nwaves) {
+#pragma unroll
+  for (int m = 0; m < M; m++) v[m] = wave_sum(v[m]);
+  __syncthreads();
+  if (lane_id() == 0) {
+#pragma unroll
+    for (int m = 0; m < M; m++) red[m * GEMV_MAX_WAVES + (threadIdx.x >> 6)] = v[m];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; m++) {
+    float t = 0.0f;
+#pragma unroll
+    for (int i = 0; i < GEMV_MAX_WAVES; i++) {
+      const float r = red[m * GEMV_MAX_WAVES + i];
+      t += i < nwaves ? r : 0.0f;
+    }
+    v[m] = t;
+  }
+}
+
 #define XREG 16   /* x elements per thread kept in registers by the staging */
 
 // the output stage of one row group (one lane, wave-uniform values)
@@ -280,14 +304,16 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   const char *wb = (const char *)a.w;
 
   // ---- 1. loads in flight before any arithmetic ----
-  // Each wave's loads return in issue order.  Standalone at M = 1 with 16-bit
-  // x: x and a fused norm's gain / bias vectors are issued first, then the
-  // first weight batch, so the staging and the norm's block reductions run
-  // while the weights are in flight (measured on gfx950: 1.2-1.3 us less per
-  // fused-norm launch at the C4 shapes; no change without a norm; f32 x
-  // measured slower).  With more rows (x would hold too many registers across
-  // the weight loads) and in the persistent kernel (COH: x is written by other
-  // blocks of the launch and is read only after wait()), the weights go first.
+  // Each wave's loads return in issue order.  Standalone with 16-bit x: all M
+  // rows of x and a fused norm's gain / bias vectors are issued first, then
+  // the first weight batch, so the staging and the norm's block reductions run
+  // while the weights are in flight (measured on gfx950 at M = 1: 1.2-1.3 us
+  // less per fused-norm launch at the C4 shapes; no change without a norm; f32
+  // x measured slower).  Row by row after the weights, as M > 1 had been, each
+  // row's loads waited for every load before them: at M = 3 the fused-norm
+  // gate/up (28672 x 4096 fp8) took 39.3 us against 30.6 now.  In the persistent
+  // kernel (COH: x is written by other blocks of the launch and is read only
+  // after wait()) the weights go first.
   // The weight loads of row group gg, chunk batch c0: raw buffer loads
   // through a resource over the group's rows, so a row past N or a chunk past
   // C reads zero by the hardware range check with no memory access and every
@@ -322,12 +348,14 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   // buffer loads, an operand the epilogue does not use reads zero through an
   // empty range; the RoPE pair follows once the position is back (after x
   // staging).  Values only: the epilogue's arithmetic is unchanged.
-  constexpr bool PRE = !COH;
+  // (not at M = 4: 18 values held across the loop spilled, and a reload from
+  // scratch in the loop waits for every weight load in flight)
+  constexpr bool PRE = !COH && M <= 3;
   EpiPre<R, M> pre;
   uint32_t pre_len = 0;
   const bool pre_qkv = a.epi == THVM_EPI_QKV || a.epi == THVM_EPI_QKV_ROPE;
   const uint32_t pre_n0 = (g < G ? g : 0u) * R;
-  if (PRE) {
+  auto load_pre = [&] {
     const buf_t rsc = buf_rsrc(a.scale, a.scale ? N * 4u : 0u);
 #pragma unroll
     for (int r = 0; r < R; r++) pre.sc[r] = buf_ld4(rsc, (pre_n0 + r) * 4u);
@@ -346,19 +374,36 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       }
     const buf_t rls = buf_rsrc(a.len, pre_qkv ? 4u : 0u);
     pre_len = buf_ld4(rls, 0);
-  }
+  };
+  // (M rows of them are requested after x is staged: beside x, its gains and the
+  // weights in flight they would not fit in 128 registers)
+  if (PRE && M == 1) load_pre();
   const uint32_t NVt = K / VE;           // x vectors per row
   // (with a fused norm, threads at or beyond nthr take no part in the staging
   // but join its block barriers: the norm's reduction order is that of an
   // nthr-thread block)
   const uint32_t tid = threadIdx.x < nthr ? threadIdx.x : NVt;
-  constexpr int XN = 4;                  // no norm: x vectors per thread per staging pass
-  constexpr int NVN = XREG / VE;         // fused norm: x vectors per thread
-  constexpr int NPRE = XN > NVN ? XN : NVN;
-  // x row 0 as raw 16-byte vectors (!COH): the norm path's vectors tid + j*nthr,
-  // or the no-norm path's first pass threadIdx.x + j*bdim (clamped
-  // indices; out-of-row vectors are never stored)
-  constexpr bool XPRE = !COH && M == 1 && XD != XD_F32 && XD != XD_SUM4;
+  constexpr int XN = 4;                  // no norm: x vectors of a row per thread and staging pass
+  constexpr int XNM = M == 1 ? XN : 8;   // the same for several rows, standalone: of the rows taken as one list
+  constexpr int NVN = XREG / VE;         // fused norm: x vectors per thread and row
+  // rows normed per pass: all, but two at a time at M = 4 (four rows of x beside
+  // the gains and the weights in flight spilled)
+  constexpr int MP = M == 4 ? 2 : M;
+  constexpr int NPRE = XNM > MP * NVN ? XNM : MP * NVN;
+  // x as raw 16-byte vectors, requested before the weights: with a norm, row
+  // m's vectors tid + j*nthr at [m*NVN + j]; without, the first pass over the
+  // rows' list, vectors threadIdx.x + j*bdim (clamped indices; vectors past
+  // the rows are never stored)
+  constexpr bool XPRE = !COH && XD != XD_F32 && XD != XD_SUM4;
+  const uint32_t NVM = (uint32_t)M * NVt;
+  // vector f of the rows' list -> its row and its vector there
+  auto row_of = [&](uint32_t f, uint32_t &v) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 1; i < M; i++) m += f >= (uint32_t)i * NVt ? 1u : 0u;
+    v = f - m * NVt;
+    return m;
+  };
   // summed x: thread t's element pairs 2 (t + j bdim) of the four quarters
   // and their gains, requested before the weights (8-byte unguarded loads)
   constexpr bool XSUM = XD == XD_SUM4;
@@ -377,16 +422,26 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   }
   uint4 xpre[NPRE];
   if (XPRE) {
-    const char *x0 = (const char *)xrow(0);
+    // (uniform skips of vectors past the rows for every thread: a K below the
+    // staging's reach needs fewer loads)
+    if (a.norm == 0) {
 #pragma unroll
-    for (int j = 0; j < NPRE; j++) {
-      // (a uniform skip of vectors past the row for every thread: K below
-      // the staging's reach needs fewer loads)
-      const uint32_t stride = a.norm == 0 ? bdim : nthr;
-      if ((a.norm == 0 ? j >= XN : j >= NVN) || j * stride >= NVt) break;
-      const uint32_t v = (a.norm == 0 ? threadIdx.x : tid) + j * stride;
-      const uint32_t vc = v < NVt ? v : 0;
-      xpre[j] = ld16(x0 + (uint64_t)vc * VE * XDr<XD>::B);
+      for (int j = 0; j < XNM; j++) {
+        if (j * bdim >= NVM) break;
+        const uint32_t f = threadIdx.x + j * bdim;
+        uint32_t v;
+        const uint32_t m = row_of(f < NVM ? f : 0u, v);
+        xpre[j] = ld16((const char *)xrow((int)m) + (uint64_t)v * VE * XDr<XD>::B);
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < MP; m++)
+#pragma unroll
+        for (int j = 0; j < NVN; j++) {
+          if (j * nthr >= NVt) break;
+          const uint32_t v = tid + j * nthr, vc = v < NVt ? v : 0;
+          xpre[m * NVN + j] = ld16((const char *)xrow(m) + (uint64_t)vc * VE * XDr<XD>::B);
+        }
     }
   }
   // a fused norm's gain (and LayerNorm bias) vectors: loaded with the first
@@ -403,8 +458,10 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       for (int i = 0; i < VE; i += 4) {
         const float4 t = hw ? *(const float4 *)(a.norm_w + vc * VE + i) : make_float4(1.f, 1.f, 1.f, 1.f);
         gw[j][i] = t.x; gw[j][i + 1] = t.y; gw[j][i + 2] = t.z; gw[j][i + 3] = t.w;
-        const float4 u = hb ? *(const float4 *)(a.norm_b + vc * VE + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-        gb[j][i] = u.x; gb[j][i + 1] = u.y; gb[j][i + 2] = u.z; gb[j][i + 3] = u.w;
+        if (M == 1 || COH) {
+          const float4 u = hb ? *(const float4 *)(a.norm_b + vc * VE + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+          gb[j][i] = u.x; gb[j][i + 1] = u.y; gb[j][i + 2] = u.z; gb[j][i + 3] = u.w;
+        }
       }
     }
   };
@@ -445,10 +502,109 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       const uint32_t hi = e < K ? xs_index<XT, E>(K, C, 0, e) : K;
       *(uint32_t *)(xs_raw + (size_t)hi * 2u) = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
     }
+  } else if constexpr (!COH && M > 1) {
+    if (a.norm == 0) {
+      // no reduction: every thread of the block stages, XNM vectors of x in
+      // flight per thread before the first LDS store
+      for (uint32_t f0 = threadIdx.x; f0 < NVM; f0 += XNM * bdim) {
+        uint4 q[XNM];
+        const bool first = f0 == threadIdx.x;
+#pragma unroll
+        for (int j = 0; j < XNM; j++) {
+          const uint32_t f = f0 + j * bdim;
+          if (f < NVM) {
+            uint32_t v;
+            const uint32_t m = row_of(f, v);
+            q[j] = XPRE && first ? xpre[j] : xraw<XD, false>(xrow((int)m), (uint64_t)v * VE);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < XNM; j++) {
+          const uint32_t f = f0 + j * bdim;
+          if (f < NVM) {
+            uint32_t v;
+            const uint32_t m = row_of(f, v);
+            xs_put_raw<XD, XT, E>(xs_raw, K, C, m, v, q[j]);
+          }
+        }
+      }
+    } else
+#pragma unroll
+    for (int mb = 0; mb < M; mb += MP) {
+#pragma unroll
+      for (int m = 0; m < MP; m++)
+#pragma unroll
+        for (int j = 0; j < NVN; j++) {
+          const uint32_t v = tid + j * nthr;
+          if ((!XPRE || mb > 0) && v < NVt) xpre[m * NVN + j] = xraw<XD, false>(xrow(mb + m), (uint64_t)v * VE);
+          if (v >= NVt) xpre[m * NVN + j] = make_uint4(0, 0, 0, 0);   // decodes to zeros
+        }
+      // (each pass decodes the raw vectors again: kept as floats across the
+      // passes, M rows spilled)
+      auto hold = [&] {
+#pragma unroll
+        for (int i = 0; i < MP * NVN; i++)
+          asm volatile("" : "+v"(xpre[i].x), "+v"(xpre[i].y), "+v"(xpre[i].z), "+v"(xpre[i].w));
+      };
+      const float invK = 1.0f / (float)K;
+      float mean[MP], s2[MP];
+#pragma unroll
+      for (int m = 0; m < MP; m++) mean[m] = s2[m] = 0.0f;
+      if (a.norm == 2) {
+#pragma unroll
+        for (int m = 0; m < MP; m++)
+#pragma unroll
+          for (int j = 0; j < NVN; j++) {
+            float xf[VE];
+            xdec<XD>(xpre[m * NVN + j], xf);
+#pragma unroll
+            for (int i = 0; i < VE; i++) mean[m] += xf[i];
+            }
+        block_sum_m<MP>(mean, red, nw);
+#pragma unroll
+        for (int m = 0; m < MP; m++) mean[m] = mean[m] * invK;
+        hold();
+      }
+#pragma unroll
+      for (int m = 0; m < MP; m++)
+#pragma unroll
+        for (int j = 0; j < NVN; j++) {
+          const bool vok = tid + j * nthr < NVt;
+          float xf[VE];
+          xdec<XD>(xpre[m * NVN + j], xf);
+#pragma unroll
+          for (int i = 0; i < VE; i++) {
+            const float d = xf[i] - mean[m];
+            s2[m] += vok ? d * d : 0.0f;
+          }
+        }
+      block_sum_m<MP>(s2, red, nw);
+      hold();
+#pragma unroll
+      for (int m = 0; m < MP; m++) {
+        const float inv = 1.0f / sqrtf(s2[m] * invK + a.norm_eps);
+#pragma unroll
+        for (int j = 0; j < NVN; j++) {
+          const uint32_t v = tid + j * nthr;
+          if (v < NVt) {
+            float val[VE];
+            xdec<XD>(xpre[m * NVN + j], val);
+#pragma unroll
+            for (int i = 0; i < VE; i++) {
+              // (x - mean) * inv * w (+ b), the norm kernel's own formula
+              val[i] = (val[i] - mean[m]) * inv;
+              if (a.norm_w) val[i] = val[i] * gw[j][i];
+              if (a.norm == 2 && a.norm_b) val[i] = val[i] + a.norm_b[v * VE + i];
+            }
+            xs_put_f<XD, XT, E>(xs_raw, K, C, mb + m, v, val);
+          }
+        }
+      }
+    }
   } else
   for (int m = 0; m < M; m++) {
     const void *xr = xrow(m);
-    const bool pre = XPRE && m == 0;     // row 0 already in xpre
+    constexpr bool pre = XPRE;           // (M = 1) the row is already in xpre
     if (a.norm == 0) {
       // no reduction: every thread of the block stages, XN vectors of x in
       // flight per thread before the first LDS store
@@ -516,6 +672,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       }
     }
   }
+  if (PRE && M > 1) load_pre();
   __syncthreads();
   pclk(clk, a.clk_cap, 2);
   if (PRE) {   // the position is back (loaded first): the RoPE pair's loads

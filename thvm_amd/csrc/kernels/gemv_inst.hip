@@ -13,10 +13,15 @@
 // blockIdx.y selects a chunk of M batch rows (x, y and res advance by M rows
 // per chunk): batches above 4 rows whose operands the MFMA GEMM does not take
 // run as chunks of 4, each output row computed exactly as at M <= 4.
+// More than one x row: blocks of at most 8 waves, two per CU (128 VGPRs), with
+// fewer chunks in flight as the rows' staging and sums take the registers
+// (pick_m): 28672 x 4096 fp8 with a fused norm, us before / now: M = 2 31.2 /
+// 25.5, M = 3 39.3 / 30.6, M = 4 44.8 / 35.5 (M = 4 with the spills it has at 4
+// chunks in flight 47.9; M = 3 in one block per CU with 256 VGPRs 34.0)
 template <int WT, int XD, int M, int R, int U>
-__global__ __launch_bounds__(1024) void k_gemv(ThvmGemvArgs a) {
+__global__ __launch_bounds__(M == 1 ? 1024 : 512, 4) void k_gemv(ThvmGemvArgs a) {
   extern __shared__ __align__(16) unsigned char xs_raw[];
-  __shared__ __align__(16) float red[GEMV_MAX_WAVES];
+  __shared__ __align__(16) float red[M * GEMV_MAX_WAVES];
   const int nw = blockDim.x >> 6;
   const uint32_t g = blockIdx.x * nw + (threadIdx.x >> 6);
   if (blockIdx.y) {
@@ -39,6 +44,10 @@ __global__ __launch_bounds__(1024) void k_gemv(ThvmGemvArgs a) {
 // -------------------------------------------------------------------------
 typedef void (*gemv_fn)(ThvmGemvArgs);
 
+// U chunks per lane and row in flight.  A lane's chunk order is the same at any
+// U, so the sums are the same bits; for several rows U is what fits (4 chunks
+// of two weight rows at M = 2, 2 above: no spills), and the tuning key u only
+// chooses between 4 and 8 at one row.
 template <int WT, int XD, int R, int U>
 static gemv_fn pick_m(uint32_t M) {
   if constexpr (XD == XD_SUM4) {
@@ -46,9 +55,9 @@ static gemv_fn pick_m(uint32_t M) {
   } else {
     switch (M) {
       case 1: return k_gemv<WT, XD, 1, R, U>;
-      case 2: return k_gemv<WT, XD, 2, R, U>;
-      case 3: return k_gemv<WT, XD, 3, R, U>;
-      case 4: return k_gemv<WT, XD, 4, R, U>;
+      case 2: return k_gemv<WT, XD, 2, R, 4>;
+      case 3: return k_gemv<WT, XD, 3, R, 2>;
+      case 4: return k_gemv<WT, XD, 4, R, 2>;
       default: return nullptr;
     }
   }
