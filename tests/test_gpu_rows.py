@@ -18,7 +18,7 @@ def up(hip, a):
 
 @pytest.mark.parametrize("wdt,xdt", [(DT_FP8, DT_BF16), (DT_BF16, DT_BF16), (DT_F16, DT_F16), (DT_F32, DT_F32),
                                      (DT_FP8, DT_F32), (DT_FP8, DT_F16)])
-@pytest.mark.parametrize("N,K", [(37, 64), (2050, 1600), (130, 4096), (64, 8192), (70, 10240)])
+@pytest.mark.parametrize("N,K", [(37, 64), (2050, 1600), (130, 4096), (64, 8192), (70, 10224)])
 @pytest.mark.parametrize("norm", [0, 1, 2])
 def test_gemv_rows_equal_one_row(hip, wdt, xdt, N, K, norm):
     if norm and K > 8192:

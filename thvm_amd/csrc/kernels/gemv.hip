@@ -198,11 +198,13 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   if (U != 4 && U != 8) { snprintf(err, errlen, "gemv: u must be 4 or 8"); return -1; }
   uint32_t xsz = (a->xdt == THVM_DT_FP32 || a->wdt == THVM_DT_FP32) ? 4 : 2;
   uint64_t lds = (uint64_t)Mk * a->K * xsz + (xsum ? 16 : 0);   // (summed x: a spare word after the row)
-  if (lds > 160 * 1024) {
+  const uint64_t red = a->norm && !xsum ? (uint64_t)Mk * GEMV_MAX_WAVES * 4 : 0;   // the norm's partial sums
+  if (lds + (red ? red : GEMV_MAX_WAVES * 4) > 160 * 1024) {
     snprintf(err, errlen, "gemv: M*K=%llu x elements exceed LDS (use the MFMA GEMM)",
              (unsigned long long)Mk * a->K);
     return -1;
   }
+  lds += red;
   gemv_fn f = nullptr;
   switch (a->wdt) {
     case THVM_DT_FP32: f = pick_x<WT_F32>(a->xdt, Mk, R, U); break;

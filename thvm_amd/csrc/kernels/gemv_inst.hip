@@ -21,7 +21,9 @@
 template <int WT, int XD, int M, int R, int U>
 __global__ __launch_bounds__(M == 1 ? 1024 : 512, 4) void k_gemv(ThvmGemvArgs a) {
   extern __shared__ __align__(16) unsigned char xs_raw[];
-  __shared__ __align__(16) float red[M * GEMV_MAX_WAVES];
+  // a fused norm's partial sums, after the rows (the launcher adds the room)
+  constexpr uint32_t XB = WT == WT_F32 || XD == XD_F32 ? 4 : 2;
+  float *const red = (float *)(xs_raw + (size_t)M * a.K * XB);
   const int nw = blockDim.x >> 6;
   const uint32_t g = blockIdx.x * nw + (threadIdx.x >> 6);
   if (blockIdx.y) {
