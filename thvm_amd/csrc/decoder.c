@@ -559,13 +559,15 @@ static int op_tail(Decoder *d, u32 lm_w, u32 lm_s, const NormSpec *fn) {
     return op_add(d, "spec_accept", p, e, 5);
   }
   char sk[96];
-  snprintf(p, sizeof p, "thvm-builtin:argmax b=%u v=%u nb=%u hist=1 hstride=%u%s", c->batch,
-           c->vocab, nb, c->max_seq + 1, sample_keys(c, sk, sizeof sk));
+  /* a greedy step's argmax also advances the length; sampling keeps the launch */
+  const int bump = c->temperature == 0.0f;
+  snprintf(p, sizeof p, "thvm-builtin:argmax b=%u v=%u nb=%u hist=1 hstride=%u bump=%d%s", c->batch,
+           c->vocab, nb, c->max_seq + 1, bump, sample_keys(c, sk, sizeof sk));
   u32 b[6] = {tens_find(d, "tok"), tens_find(d, "logits"), tens_find(d, "am.pv"),
               tens_find(d, "am.pi"), tens_find(d, "hist"), tens_find(d, "len")};
   if (op_add(d, "argmax", p, b, 6)) return -1;
   u32 L = tens_find(d, "len");
-  return op_add(d, "len_bump", "thvm-builtin:len_bump delta=1", &L, 1);
+  return bump ? 0 : op_add(d, "len_bump", "thvm-builtin:len_bump delta=1", &L, 1);
 }
 
 /* The persistent step (step_mode 1): the same weights and state as the op
@@ -1179,12 +1181,13 @@ static int build_dsv2(Decoder *d) {
   if (op_add(d, "lm_head", p, la, ln)) return -1;
   const u32 nb = V >= 256 * 64 ? 256 : (V + 63) / 64;
   char sk[96];
-  snprintf(p, sizeof p, "thvm-builtin:argmax b=%u v=%u nb=%u hist=1 hstride=%u%s", B, V, nb,
-           c->max_seq + 1, sample_keys(c, sk, sizeof sk));
+  const int bump = c->temperature == 0.0f;
+  snprintf(p, sizeof p, "thvm-builtin:argmax b=%u v=%u nb=%u hist=1 hstride=%u bump=%d%s", B, V, nb,
+           c->max_seq + 1, bump, sample_keys(c, sk, sizeof sk));
   u32 am[6] = {tens_find(d, "tok"), tens_find(d, "logits"), tens_find(d, "am.pv"),
                tens_find(d, "am.pi"), tens_find(d, "hist"), L};
   if (op_add(d, "argmax", p, am, 6)) return -1;
-  const int rc = op_add(d, "len_bump", "thvm-builtin:len_bump delta=1", &L, 1);
+  const int rc = bump ? 0 : op_add(d, "len_bump", "thvm-builtin:len_bump delta=1", &L, 1);
   d->cur_tag = -1;
   return rc;
 }

@@ -511,7 +511,8 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
     NEED(spec_u32(&sp, "b", &a.B, 1, 0) || spec_u32(&sp, "v", &a.V, 1, 0) ||
          spec_u32(&sp, "nb", &a.nb, 0, 256) || spec_u32(&sp, "hist", &hist, 0, 0) ||
          spec_u32(&sp, "hstride", &a.hist_stride, 0, 0) || spec_f32(&sp, "temp", &temp, 0, 0.0f) ||
-         spec_u64(&sp, "seed", &a.seed, 0, 0));
+         spec_u64(&sp, "seed", &a.seed, 0, 0) || spec_u32(&sp, "bump", &a.bump, 0, 0));
+    if (a.bump && (!hist || temp > 0.0f)) { hb_set_error("builtin argmax: bump=1 needs hist=1 and temp=0"); return -1; }
     if (!(temp >= 0.0f) || temp > 1e30f) { hb_set_error("builtin argmax: temp must be >= 0"); return -1; }
     a.inv_temp = temp > 0.0f ? 1.0f / temp : 0.0f;
     if (a.nb > a.V) a.nb = a.V;

@@ -318,6 +318,7 @@ typedef struct ThvmArgmaxArgs {
                             * instead of the argmax (pi then holds f32 block
                             * sums); the draw is keyed on (seed, row, len[0]) */
   uint64_t seed;
+  uint32_t bump;           /* greedy only: also len[0] += 1, last             */
 } ThvmArgmaxArgs;
 int thvm_k_argmax(const ThvmArgmaxArgs *a, hipStream_t s, char *err, int errlen);
 

@@ -105,7 +105,11 @@ __global__ __launch_bounds__(ATT_THREADS) void k_attn_fused(ThvmAttnArgs a) {
   const int wv = threadIdx.x >> 6;
   AttnSplit<HD, G, AT, true, false> u;
   u.issue(a, kvh, split, b, wv, L);
-  u.finish(a, kvh, split, b, wv, threadIdx.x, L, true, s);
+  // a row of one live split needs no hand-off: its unit writes the output, the
+  // same bits without the drain, the atomic and the partial's round trip
+  // (GPT-2 small at 17..32 rows, 12 heads: DIRECT_OLD us per launch)
+  u.template finish<true>(a, kvh, split, b, wv, threadIdx.x, L, true, s, n_live == 1);
+  if (n_live == 1) return;                         // block-uniform
   attn_handoff_merge<HD, G, AT>(a, b, kvh, n_live, &last, &ms);
 }
 
@@ -132,6 +136,7 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void k_attn_multi(ThvmAttnArgs a) {
   const int32_t L = attn_row_len(a, b);
   const uint32_t cpb = a.cpb, c0 = grp * cpb;
   if ((int32_t)(c0 * ATT_CHUNK) >= L) return;      // the merge reads only live partials
+  const bool alone = FUSE && attn_live(a, L) == 1; // (as in k_attn_fused: no hand-off)
   // phase clock: 0 entry, 1 first chunk's loads issued and q decoded, 2 first
   // chunk consumed, 3 chunks done, 4 row groups combined, 5 wave maxima in
   // LDS, 6 wave accumulators in LDS, 7 partial stored (drained)
@@ -291,6 +296,10 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void k_attn_multi(ThvmAttnArgs a) {
       sv += s.wacc[w][g][d] * f;
       lt += f * s.wl[w][g];
     }
+    if (FUSE && alone) {
+      st_act<AT, false>(a.out, ((uint64_t)b * a.H + kvh * G + g) * HD + d, sv * (lt > 0.0f ? 1.0f / lt : 0.0f));
+      continue;
+    }
     const uint64_t pi = (((uint64_t)b * a.H + kvh * G + g) * a.n_split + grp) * (HD + 2);
     if (FUSE) {
       coh_stf(a.part, (uint32_t)((pi + d) * 4), sv);
@@ -301,7 +310,7 @@ __global__ __launch_bounds__(ATT_THREADS, 4) void k_attn_multi(ThvmAttnArgs a) {
       if (d == 0) { pp[HD] = M; pp[HD + 1] = lt; }
     }
   }
-  if (FUSE) attn_handoff_merge<HD, G, AT>(a, b, kvh, attn_live(a, L), &last, &ms);
+  if (FUSE && !alone) attn_handoff_merge<HD, G, AT>(a, b, kvh, attn_live(a, L), &last, &ms);
   pclk_end(a.clk, a.clk_cap);
 }
 

@@ -156,9 +156,12 @@ struct AttnSplit {
   // Scores, softmax and the V mix of the unit; writes the split's partial.
   // Every thread of the block calls it (the two block barriers inside are
   // block-wide); `active` false skips the work.
+  // DIRECT: the unit is its row's only live one and writes the output row itself
+  // (the merge of a single partial: its acc / l).
+  template <bool DIRECT = false>
   __device__ __forceinline__ void finish(const ThvmAttnArgs &a, uint32_t kvh, uint32_t split,
                                          uint32_t b, int wv, int tid, int32_t L, bool active,
-                                         AttnLds<HD, G> &s) {
+                                         AttnLds<HD, G> &s, bool direct = false) {
     const int lane = lane_id();
     const int rg = lane / LPR, li = lane % LPR;
     const uint32_t d0 = li * EPL;
@@ -264,6 +267,10 @@ struct AttnSplit {
           const float f = mwv == -INFINITY ? 0.0f : fexp2(mwv - M);
           sv += s.wacc[w][g][d] * f;
           l += f * s.wl[w][g];
+        }
+        if (DIRECT && direct) {
+          st_act<AT, false>(a.out, ((uint64_t)b * a.H + kvh * G + g) * HD + d, sv * (l > 0.0f ? 1.0f / l : 0.0f));
+          continue;
         }
         const uint64_t pi = (((uint64_t)b * a.H + kvh * G + g) * a.n_split + split) * (HD + 2);
         if (COH) {

@@ -178,6 +178,14 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   if (!a->tune_r && R == 1 && a->N % 2 == 0 && a->N > 2048 && a->M <= 4 && (uint64_t)a->K * wsz / 16 <= 128) {
     R = 2;
   }
+  // two rows per wave too where one per wave takes more than 256 blocks of 8
+  // waves and two fit in 256, over rows of less than a full batch of chunks: one
+  // block per CU (3072 x 768 f32 with a LayerNorm: 6.96 -> 6.25 us with the wave
+  // count below; full-batch rows, 4096 x 4096 fp8, are faster at 16 waves)
+  if (!a->tune_r && R == 1 && a->M == 1 && a->N % 2 == 0 && a->N > 2048 && a->N <= 4096 &&
+      (uint64_t)a->K * wsz / 16 < 256 && a->norm != 1) {
+    R = 2;
+  }
   // three or four x rows over long weight rows (>= 768 chunks): two rows per
   // wave share each x read from LDS (measured on gfx950 at the C4 down shape,
   // 14336-wide fp8 rows: M = 3 21.2 -> 17.1 us, M = 4 23.3 -> 18.8; at M = 2 one
@@ -229,6 +237,16 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   if (!a->tune_waves && Mk == 1 && chunks == 1 && (uint64_t)a->K * wsz / 16 == 64u * (uint32_t)U &&
       (Gr + 7) / 8 > 256 && (Gr + 15) / 16 <= 256) {
     waves = (Gr + 255) / 256;
+  }
+  // fewer than 8 waves where that still is one block per CU or less: the rows
+  // spread over every CU (768 x 3072 f32, 96 blocks of 8 waves: 6.02 -> 5.65 us
+  // at 3; 2304 x 768 with a LayerNorm in pairs, 144 blocks: 6.52 -> 5.64 at 6).
+  // Not with a fused RMSNorm, whose sum is in the order of a 512-thread block
+  // (the persistent step's).
+  if (!a->tune_waves && Mk == 1 && chunks == 1 && !xsum && a->norm != 1 && Gr <= 2048) {
+    const uint32_t w = (Gr + 255) / 256, wmin = a->norm ? (uint32_t)((a->K + XREG * 64 - 1) / (XREG * 64)) : 1u;
+    const uint32_t lo = wmin > 3 ? wmin : 3;
+    waves = w < lo ? lo : w > 8 ? 8 : w;
   }
   if (Mk > 1 && waves > 8) waves = 8;   // the instances' block limit; the sums do not depend on it
   if (xsum && a->K > 2u * GEMV_SQ * 64u * waves) {   // the staging's element pairs per thread

@@ -327,9 +327,23 @@ __device__ __forceinline__ bool am_better(float v, int32_t i, float bv, int32_t 
   return v > bv || (v == bv && i < bi);
 }
 
+// the wave's best (value, lowest index): the value by a DPP max, the index by a
+// DPP min over the lanes that hold it
+__device__ __forceinline__ void am_wave(float &bv, int32_t &bi) {
+  const float m = wave_max(bv);
+  int32_t i = bv == m ? bi : 0x7fffffff;
+#define AM_MIN(CTRL, RM) i = min(i, __builtin_amdgcn_update_dpp(i, i, CTRL, RM, 0xf, false))
+  AM_MIN(0xB1, 0xf); AM_MIN(0x4E, 0xf); AM_MIN(0x141, 0xf); AM_MIN(0x140, 0xf); AM_MIN(0x142, 0xa); AM_MIN(0x143, 0xc);
+#undef AM_MIN
+  bv = m;
+  bi = __builtin_amdgcn_readlane(i, 63);
+}
+
+// four waves per block: a wave reduction each and one barrier (a shared-memory
+// tree over the 256 threads took eight)
 __global__ __launch_bounds__(256) void k_argmax_part(ThvmArgmaxArgs a) {
-  __shared__ float sv[256];
-  __shared__ int32_t si[256];
+  __shared__ float sv[4];
+  __shared__ int32_t si[4];
   const uint32_t b = blockIdx.y, blk = blockIdx.x, t = threadIdx.x;
   const uint32_t chunk = (a.V + a.nb - 1) / a.nb;
   const uint64_t lo = (uint64_t)blk * chunk;
@@ -342,41 +356,42 @@ __global__ __launch_bounds__(256) void k_argmax_part(ThvmArgmaxArgs a) {
     float x = lg[i];
     if (am_better(x, (int32_t)i, bv, bi)) { bv = x; bi = (int32_t)i; }
   }
-  sv[t] = bv; si[t] = bi;
+  am_wave(bv, bi);
+  if ((t & 63) == 0) { sv[t >> 6] = bv; si[t >> 6] = bi; }
   __syncthreads();
-  for (uint32_t st = 128; st > 0; st >>= 1) {
-    if (t < st && am_better(sv[t + st], si[t + st], sv[t], si[t])) {
-      sv[t] = sv[t + st]; si[t] = si[t + st];
-    }
-    __syncthreads();
-  }
-  if (t == 0) { a.pv[b * a.nb + blk] = sv[0]; a.pi[b * a.nb + blk] = si[0]; }
+  if (t != 0) return;
+#pragma unroll
+  for (int w = 1; w < 4; w++)
+    if (am_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
+  a.pv[b * a.nb + blk] = bv;
+  a.pi[b * a.nb + blk] = bi;
 }
 
-// one wave per batch row: lanes scan the block partials, then a shuffle
-// reduction keeps (max value, lowest index)
-__global__ void k_argmax_fin(ThvmArgmaxArgs a) {
-  const uint32_t b = blockIdx.x;
+// One block, a wave per batch row: lanes scan the block partials, then a wave
+// reduction keeps (max value, lowest index).  bump: the block also advances the
+// length once every row has written its id, in place of a launch of its own
+// (1.6 us of a graph's step for one add).
+#define AM_FIN_WAVES 16
+__global__ __launch_bounds__(64 * AM_FIN_WAVES) void k_argmax_fin(ThvmArgmaxArgs a) {
   const int lane = lane_id();
-  float bv = -INFINITY;
-  int32_t bi = 0x7fffffff;
-  for (uint32_t k = lane; k < a.nb; k += 64) {
-    float v = a.pv[b * a.nb + k];
-    int32_t i = a.pi[b * a.nb + k];
-    if (am_better(v, i, bv, bi)) { bv = v; bi = i; }
+  const int32_t L = a.len ? a.len[0] : 0;
+  for (uint32_t b = threadIdx.x >> 6; b < a.B; b += blockDim.x >> 6) {
+    float bv = -INFINITY;
+    int32_t bi = 0x7fffffff;
+    for (uint32_t k = lane; k < a.nb; k += 64) {
+      const float v = a.pv[b * a.nb + k];
+      const int32_t i = a.pi[b * a.nb + k];
+      if (am_better(v, i, bv, bi)) { bv = v; bi = i; }
+    }
+    am_wave(bv, bi);
+    if (lane == 0) {
+      a.tok[b] = bi;
+      if (a.hist && L >= 0 && (uint32_t)L < a.hist_stride) a.hist[(uint64_t)b * a.hist_stride + L] = bi;
+    }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(bv, off);
-    int32_t oi = __shfl_xor(bi, off);
-    if (am_better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-  }
-  if (lane != 0) return;
-  a.tok[b] = bi;
-  if (a.hist) {
-    int32_t L = a.len[0];
-    if (L >= 0 && (uint32_t)L < a.hist_stride) a.hist[(uint64_t)b * a.hist_stride + L] = bi;
-  }
+  if (!a.bump) return;
+  __syncthreads();                                 // every wave has read the length
+  if (threadIdx.x == 0) *(int32_t *)a.len = L + 1;
 }
 
 // ---- temperature sampling: id ~ softmax(logits / T), replacing argmax ----
@@ -537,7 +552,8 @@ __global__ __launch_bounds__(64) void k_sample_fin(ThvmArgmaxArgs a) {
 #pragma clang fp contract(fast)   // back to the HIP default for the rest of the file
 
 extern "C" int thvm_k_argmax(const ThvmArgmaxArgs *a, hipStream_t s, char *err, int errlen) {
-  if (a->B == 0 || a->V == 0 || a->nb == 0 || a->nb > a->V || (a->hist && !a->len)) {
+  if (a->B == 0 || a->V == 0 || a->nb == 0 || a->nb > a->V || (a->hist && !a->len) ||
+      (a->bump && (!a->len || a->inv_temp > 0.0f))) {
     snprintf(err, errlen, "argmax: bad args");
     return -1;
   }
@@ -553,7 +569,7 @@ extern "C" int thvm_k_argmax(const ThvmArgmaxArgs *a, hipStream_t s, char *err, 
     return 0;
   }
   thvm_launch(true, false, k_argmax_part, dim3(a->nb, a->B), dim3(256), 0, s, *a);
-  thvm_launch(false, true, k_argmax_fin, dim3(a->B), dim3(64), 0, s, *a);
+  thvm_launch(false, true, k_argmax_fin, dim3(1), dim3(64 * (a->B < AM_FIN_WAVES ? a->B : AM_FIN_WAVES)), 0, s, *a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { snprintf(err, errlen, "argmax launch: %s", hipGetErrorString(e)); return -1; }
   return 0;
