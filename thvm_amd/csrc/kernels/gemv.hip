@@ -189,8 +189,9 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   // three or four x rows over long weight rows (>= 768 chunks): two rows per
   // wave share each x read from LDS (measured on gfx950 at the C4 down shape,
   // 14336-wide fp8 rows: M = 3 21.2 -> 17.1 us, M = 4 23.3 -> 18.8; at M = 2 one
-  // row is faster, 14.0 against 15.8); bit-identical sums
-  if (!a->tune_r && R == 1 && Mk >= 3 && a->N % 2 == 0 && (uint64_t)a->K * wsz / 16 >= 768) R = 2;
+  // row is faster, 14.0 against 15.8, and so it is with f32 operands, 768 x 3072
+  // at M = 3 7.2 against 10.6); bit-identical sums
+  if (!a->tune_r && R == 1 && Mk >= 3 && a->xdt != THVM_DT_FP32 && a->wdt != THVM_DT_FP32 && a->N % 2 == 0 && (uint64_t)a->K * wsz / 16 >= 768) R = 2;
   if (a->tune_r) {
     if (a->tune_r != 1 && a->tune_r != 2) { snprintf(err, errlen, "gemv: r must be 1 or 2"); return -1; }
     if ((pairs && a->tune_r == 1) || a->N % a->tune_r) { snprintf(err, errlen, "gemv: r=%u does not tile N/epilogue", a->tune_r); return -1; }

@@ -304,12 +304,13 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   const char *wb = (const char *)a.w;
 
   // ---- 1. loads in flight before any arithmetic ----
-  // Each wave's loads return in issue order.  Standalone with 16-bit x: all M
-  // rows of x and a fused norm's gain / bias vectors are issued first, then
-  // the first weight batch, so the staging and the norm's block reductions run
-  // while the weights are in flight (measured on gfx950 at M = 1: 1.2-1.3 us
-  // less per fused-norm launch at the C4 shapes; no change without a norm; f32
-  // x measured slower).  Row by row after the weights, as M > 1 had been, each
+  // Each wave's loads return in issue order.  Standalone: all M rows of x and
+  // a fused norm's gain / bias vectors are issued first, then the first weight
+  // batch, so the staging and the norm's block reductions run while the weights
+  // are in flight (measured on gfx950 at M = 1: 1.2-1.3 us less per fused-norm
+  // launch at the C4 shapes, f32 3072 x 768 with a LayerNorm 6.3 -> 5.4; no
+  // change without a norm).  Not f32 x of two or three rows: with twice the
+  // registers per row they spill.  Row by row after the weights, as M > 1 had been, each
   // row's loads waited for every load before them: at M = 3 the fused-norm
   // gate/up (28672 x 4096 fp8) took 39.3 us against 30.6 now.  In the persistent
   // kernel (COH: x is written by other blocks of the launch and is read only
@@ -376,7 +377,8 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
     pre_len = buf_ld4(rls, 0);
   };
   // (M rows of them are requested after x is staged: beside x, its gains and the
-  // weights in flight they would not fit in 128 registers)
+  // weights in flight they would not fit in 128 registers; the position alone up
+  // front spilled at M = 3, a layer at batch 3 89.8 -> 92.2 us)
   if (PRE && M == 1) load_pre();
   const uint32_t NVt = K / VE;           // x vectors per row
   // (with a fused norm, threads at or beyond nthr take no part in the staging
@@ -394,7 +396,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   // m's vectors tid + j*nthr at [m*NVN + j]; without, the first pass over the
   // rows' list, vectors threadIdx.x + j*bdim (clamped indices; vectors past
   // the rows are never stored)
-  constexpr bool XPRE = !COH && XD != XD_F32 && XD != XD_SUM4;
+  constexpr bool XPRE = !COH && (XD != XD_F32 || M == 1 || M == 4) && XD != XD_SUM4;
   const uint32_t NVM = (uint32_t)M * NVt;
   // vector f of the rows' list -> its row and its vector there
   auto row_of = [&](uint32_t f, uint32_t &v) {

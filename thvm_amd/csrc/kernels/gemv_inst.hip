@@ -52,14 +52,17 @@ typedef void (*gemv_fn)(ThvmGemvArgs);
 // chooses between 4 and 8 at one row.
 template <int WT, int XD, int R, int U>
 static gemv_fn pick_m(uint32_t M) {
+  // (f32 weights hold a quarter of fp8's values per chunk, so one weight row per
+  // wave keeps 4: 4800 x 1600, M = 3, 15.4 us at 2)
+  constexpr int UM = WT == WT_F32 && R == 1 ? 4 : 2;
   if constexpr (XD == XD_SUM4) {
     return M == 1 ? k_gemv<WT, XD, 1, R, U> : nullptr;   // one row only
   } else {
     switch (M) {
       case 1: return k_gemv<WT, XD, 1, R, U>;
       case 2: return k_gemv<WT, XD, 2, R, 4>;
-      case 3: return k_gemv<WT, XD, 3, R, 2>;
-      case 4: return k_gemv<WT, XD, 4, R, 2>;
+      case 3: return k_gemv<WT, XD, 3, R, UM>;
+      case 4: return k_gemv<WT, XD, 4, R, UM>;
       default: return nullptr;
     }
   }
