@@ -8,7 +8,8 @@
 // [H, max_seq] score matrix become three kernels:
 //   k_mla_prep   q pe rotation, latent-row RMSNorm + k pe rotation + cache
 //                append at L-1, and qlat = q_nope . W_uk (fp8/bf16 rows, per
-//                row scale) -- one launch, blocks split between the jobs;
+//                row scale; on MFMA) -- one launch, blocks split between the
+//                jobs;
 //   k_mla_split  split-sequence flash decode: a block owns 64 cache rows of
 //                one batch row and a group of 4 heads, stages the rows in LDS
 //                once, scores the group against them (lanes split the latent
@@ -66,24 +67,151 @@ __device__ __forceinline__ float group_sum(float v, int G) {
 }
 
 // ---- k_mla_prep ---------------------------------------------------------
-// blocks [0, H*QB*BG): qlat rows (h, 64 latent rows each) for a group of
-// MLA_PREP_ROWS batch rows (BG groups); blocks [H*QB*BG, H*QB*BG + B): batch
-// row b's q pe rotation, latent norm and cache append.  256 threads.  (One
-// block per (h, 64 rows) over all 32 rows of C5 batch 32 left 160 blocks,
-// each a 32-step serial loop: 33.7 us; groups of 8 rows give 512 blocks.)
+// blocks [0, B): batch row b's latent norm and cache append; [B, 2B): its q pe
+// and k pe rotations; the rest the absorption qlat = q_nope . W_uk, each block
+// 64 latent rows of a head.  256 threads.  Latency-bound (C5 batch 32 moves 4
+// MB): what counts is the longest chain of round trips in a block.  The row
+// jobs come first and are two blocks a row: one block rotating and then
+// norming took a round trip for each, after the absorption's blocks.
+//
+// The absorption is a contraction of 16-bit q with fp8 or bf16 rows, so it
+// runs on MFMA with f32 sums: a wave owns 16 latent rows (the M side) against
+// 16 batch rows (the N side), every load of a 128-wide step of d_nope is
+// issued before the first wait, and a lane writes four consecutive latent
+// values.  The VALU form it replaces (lanes splitting d_nope, one wave sum per
+// batch row and latent row) took 11.7 us at C5 batch 32 against 4.6,
+// and 4.2 at batch 1 against 2.9; it stays for the q rows that 16-byte loads
+// cannot read (an odd row stride or rope width) and for d_nope = 8, in groups
+// of MLA_PREP_ROWS batch rows.
 #define MLA_PREP_ROWS 8
 #define MLA_PREP_PASS 4    /* W_uk row passes requested at once */
+
+// batch row b's latent row: RMSNorm over kv values, gain wkvn, append at pos
+__device__ __forceinline__ void prep_latent(const ThvmMlaArgs &a, uint32_t b, float *sm) {
+  const uint32_t kv = a.kv, qoff = a.H * (a.dn + a.dr);
+  const uint64_t qb = (uint64_t)b * a.ldq;
+  const int32_t pos = a.len[0] - 1;
+  // kv <= 512: two values and gains per thread, out before anything waits
+  const uint32_t t0 = threadIdx.x, t1 = threadIdx.x + 256, c0 = min(t0, kv - 1), c1 = min(t1, kv - 1);
+  const float v0 = bfv(a.qkv, qb + qoff + c0), v1 = bfv(a.qkv, qb + qoff + c1);
+  const float g0 = a.wkvn[c0], g1 = a.wkvn[c1];
+  float ss = 0.0f;
+  if (t0 < kv) ss += v0 * v0;
+  if (t1 < kv) ss += v1 * v1;
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  pclk(a.clk, a.clk_cap, 1);
+  if (pos < 0 || (uint32_t)pos >= a.max_seq) return;
+  float tot = 0.0f;
+  for (uint32_t w = 0; w < 4; w++) tot += sm[w];
+  const float inv = 1.0f / sqrtf(tot * (1.0f / (float)kv) + a.eps);
+  bf16_t *crow = (bf16_t *)a.ckv + ((uint64_t)b * a.max_seq + (uint32_t)pos) * kv;
+  if (t0 < kv) crow[t0] = f2bf((v0 * inv) * g0);
+  if (t1 < kv) crow[t1] = f2bf((v1 * inv) * g1);
+}
+
+// batch row b's q pe pairs (2j, 2j+1) of every head -> halves j and half + j,
+// and the same of its k pe row, appended at pos
+__device__ __forceinline__ void prep_pe(const ThvmMlaArgs &a, uint32_t b) {
+  const uint32_t H = a.H, dr = a.dr, half = dr / 2, qs = a.dn + dr;
+  const uint64_t qb = (uint64_t)b * a.ldq;
+  const int32_t pos = a.len[0] - 1;
+  if (pos < 0 || (uint32_t)pos >= a.max_seq) return;
+  bf16_t *prow = (bf16_t *)a.kpe + ((uint64_t)b * a.max_seq + (uint32_t)pos) * dr;
+  for (uint32_t i = threadIdx.x; i < (H + 1) * half; i += 256) {   // "head" H is the k pe row
+    const uint32_t h = i / half, j = i % half, base = h < H ? h * qs + a.dn : H * qs + a.kv;
+    const float xe = bfv(a.qkv, qb + base + 2 * j), xo = bfv(a.qkv, qb + base + 2 * j + 1);
+    const float c = a.rope_cos[(uint64_t)pos * half + j], sn = a.rope_sin[(uint64_t)pos * half + j];
+    bf16_t *q = h < H ? (bf16_t *)a.qpe + ((uint64_t)b * H + h) * dr : prow;
+    q[j] = f2bf(xe * c - xo * sn);
+    q[half + j] = f2bf(xo * c + xe * sn);
+  }
+}
+
+// grid 2 B + H (kv / 64) ceil(B / 16): block x's latent rows are x % (H kv /
+// 64), so the blocks that read the same W_uk rows for other batch rows lie a
+// multiple of 8 apart and share an XCD's L2.  Lane group lg holds the 16
+// values 64 step + 16 lg .. of a row as both operands' k (two MFMAs: k order
+// is free as long as A and B agree).  Every MFMA starts from zero and the
+// partial sums are added outside: chained through the accumulator, the error
+// against float64 was 6.7e-7 rms (d_nope 128, normal operands); so it is
+// 5.4e-7, as the VALU form's.
+template <bool FP8>
+__global__ __launch_bounds__(256) void k_mla_prep_mf(ThvmMlaArgs a) {
+  __shared__ float sm[4];
+  // phase clock: 0 entry, 1 latent row read (its block), 7 drained
+  pclk(a.clk, a.clk_cap, 0);
+  if (blockIdx.x < 2 * a.B) {
+    if (blockIdx.x < a.B) prep_latent(a, blockIdx.x, sm);
+    else prep_pe(a, blockIdx.x - a.B);
+    pclk_end(a.clk, a.clk_cap);
+    return;
+  }
+  const uint32_t H = a.H, dn = a.dn, kv = a.kv, QB = kv / 64, x = blockIdx.x - 2 * a.B;
+  const uint32_t hk = x % (H * QB), bt = x / (H * QB), h = hk / QB;
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  const uint32_t k0 = (hk % QB) * 64 + wv * 16, n = bt * 16 + li;      // latent rows, batch row
+  constexpr uint32_t ES = FP8 ? 1 : 2;
+  const buf_t wr = buf_rsrc((const char *)a.wuk + (uint64_t)h * kv * dn * ES, kv * dn * ES);
+  const buf_t sr = buf_rsrc(a.suk ? a.suk + (uint64_t)h * kv : nullptr, a.suk ? kv * 4u : 0u);
+  const buf_t qr = buf_rsrc(a.qkv, a.B * a.ldq * 2);
+  const uint4 sc = buf_ld16(sr, (k0 + 4 * lg) * 4u);
+  const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4_t acc = zero;
+  for (uint32_t d0 = 0; d0 < dn; d0 += 128) {
+    uint4 w[2][2], q[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const uint32_t d = d0 + 64 * u + 16 * lg;
+      const uint32_t wo = d < dn ? ((k0 + li) * dn + d) * ES : BUF_OOB;
+      const uint32_t qo = d < dn && n < a.B ? (n * a.ldq + h * (dn + a.dr) + d) * 2u : BUF_OOB;
+      w[u][0] = buf_ld16(wr, wo);
+      w[u][1] = FP8 ? make_uint4(0, 0, 0, 0) : buf_ld16(wr, wo == BUF_OOB ? BUF_OOB : wo + 16u);
+      q[u][0] = buf_ld16(qr, qo);
+      q[u][1] = buf_ld16(qr, qo == BUF_OOB ? BUF_OOB : qo + 16u);
+    }
+    f32x4_t part[4];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      uint4 a0 = w[u][0], a1 = w[u][1];
+      if (FP8) {
+        const uint4 r = w[u][0];
+        fp8x4_op<GX_BF16>(r.x, a0.x, a0.y);
+        fp8x4_op<GX_BF16>(r.y, a0.z, a0.w);
+        fp8x4_op<GX_BF16>(r.z, a1.x, a1.y);
+        fp8x4_op<GX_BF16>(r.w, a1.z, a1.w);
+      }
+      part[2 * u] = mfma16<GX_BF16>(a0, q[u][0], zero);
+      part[2 * u + 1] = mfma16<GX_BF16>(a1, q[u][1], zero);
+    }
+    acc += (part[0] + part[1]) + (part[2] + part[3]);
+  }
+  // lane: latent rows k0 + 4 lg + i of batch row n
+  if (n < a.B) {
+    float4 o = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    if (a.suk) {
+      o.x *= __uint_as_float(sc.x); o.y *= __uint_as_float(sc.y);
+      o.z *= __uint_as_float(sc.z); o.w *= __uint_as_float(sc.w);
+    }
+    *(float4 *)(a.qlat + ((uint64_t)n * H + h) * kv + k0 + 4 * lg) = o;
+  }
+  pclk_end(a.clk, a.clk_cap);
+}
+
 template <bool FP8>
 __global__ __launch_bounds__(256) void k_mla_prep(ThvmMlaArgs a) {
   extern __shared__ float sm[];
-  const uint32_t H = a.H, dn = a.dn, dr = a.dr, kv = a.kv, half = dr / 2, qs = dn + dr;
-  const uint32_t qoff = H * qs, QB = kv / 64, BG = (a.B + MLA_PREP_ROWS - 1) / MLA_PREP_ROWS;
-  const int32_t pos = a.len[0] - 1;
   // phase clock: 0 entry, 1 q nope staged (absorption blocks) or latent row
-  // read (the append block), 7 drained
+  // read (its block), 7 drained
   pclk(a.clk, a.clk_cap, 0);
-  if (blockIdx.x < H * QB * BG) {
-    const uint32_t h = blockIdx.x / (QB * BG), rem = blockIdx.x % (QB * BG);
+  if (blockIdx.x < 2 * a.B) {
+    if (blockIdx.x < a.B) prep_latent(a, blockIdx.x, sm);
+    else prep_pe(a, blockIdx.x - a.B);
+  } else {
+    const uint32_t H = a.H, dn = a.dn, kv = a.kv, qs = dn + a.dr;
+    const uint32_t QB = kv / 64, BG = (a.B + MLA_PREP_ROWS - 1) / MLA_PREP_ROWS, x = blockIdx.x - 2 * a.B;
+    const uint32_t h = x / (QB * BG), rem = x % (QB * BG);
     const uint32_t k0 = (rem / BG) * 64, b0 = (rem % BG) * MLA_PREP_ROWS;
     const uint32_t nb = min(a.B - b0, (uint32_t)MLA_PREP_ROWS);
     const uint32_t rowb = dn * (FP8 ? 1 : 2), LPR = rowb / 16;     // lanes per row
@@ -133,44 +261,6 @@ __global__ __launch_bounds__(256) void k_mla_prep(ThvmMlaArgs a) {
         }
       }
     }
-    pclk_end(a.clk, a.clk_cap);
-    return;
-  }
-  const uint32_t b = blockIdx.x - H * QB * BG;
-  if (b >= a.B || pos < 0 || (uint32_t)pos >= a.max_seq) return;
-  const uint64_t qb = (uint64_t)b * a.ldq;
-  // q pe pairs (2j, 2j+1) -> halves j and half+j, after rounding through bf16
-  for (uint32_t i = threadIdx.x; i < H * half; i += blockDim.x) {
-    const uint32_t h = i / half, j = i % half, base = h * qs + dn;
-    const float xe = bfv(a.qkv, qb + base + 2 * j), xo = bfv(a.qkv, qb + base + 2 * j + 1);
-    const float c = a.rope_cos[(uint64_t)pos * half + j], sn = a.rope_sin[(uint64_t)pos * half + j];
-    bf16_t *q = (bf16_t *)a.qpe + ((uint64_t)b * H + h) * dr;
-    q[j] = f2bf(xe * c - xo * sn);
-    q[half + j] = f2bf(xo * c + xe * sn);
-  }
-  // latent row: RMSNorm over kv values, gain wkvn, append at pos
-  float ss = 0.0f;
-  for (uint32_t t = threadIdx.x; t < kv; t += blockDim.x) {
-    const float v = bfv(a.qkv, qb + qoff + t);
-    sm[t] = v;
-    ss += v * v;
-  }
-  ss = wave_sum(ss);
-  float *red = sm + kv;
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  pclk(a.clk, a.clk_cap, 1);
-  float tot = 0.0f;
-  for (uint32_t w = 0; w < blockDim.x / 64; w++) tot += red[w];
-  const float inv = 1.0f / sqrtf(tot * (1.0f / (float)kv) + a.eps);
-  bf16_t *crow = (bf16_t *)a.ckv + ((uint64_t)b * a.max_seq + (uint32_t)pos) * kv;
-  for (uint32_t t = threadIdx.x; t < kv; t += blockDim.x) crow[t] = f2bf((sm[t] * inv) * a.wkvn[t]);
-  bf16_t *prow = (bf16_t *)a.kpe + ((uint64_t)b * a.max_seq + (uint32_t)pos) * dr;
-  for (uint32_t j = threadIdx.x; j < half; j += blockDim.x) {
-    const float xe = bfv(a.qkv, qb + qoff + kv + 2 * j), xo = bfv(a.qkv, qb + qoff + kv + 2 * j + 1);
-    const float c = a.rope_cos[(uint64_t)pos * half + j], sn = a.rope_sin[(uint64_t)pos * half + j];
-    prow[j] = f2bf(xe * c - xo * sn);
-    prow[half + j] = f2bf(xo * c + xe * sn);
   }
   pclk_end(a.clk, a.clk_cap);
 }
@@ -938,12 +1028,24 @@ extern "C" int thvm_k_mla_prep(const ThvmMlaArgs *a, hipStream_t s, char *err, i
     return -1;
   }
   const uint32_t QB = a->kv / 64, BG = (a->B + MLA_PREP_ROWS - 1) / MLA_PREP_ROWS;
-  uint64_t lds = (uint64_t)(a->B < MLA_PREP_ROWS ? a->B : MLA_PREP_ROWS) * a->dn * 4;
-  if ((uint64_t)a->kv * 4 + 64 > lds) lds = (uint64_t)a->kv * 4 + 64;
+  const uint64_t lds = (uint64_t)(a->B < MLA_PREP_ROWS ? a->B : MLA_PREP_ROWS) * a->dn * 4;   // holds the 4 wave sums too
   if (lds > 64 * 1024) { snprintf(err, errlen, "mla_prep: d_nope too large for LDS staging"); return -1; }
-  const dim3 grid(a->H * QB * BG + a->B);
-  if (a->wdt == THVM_DT_FP8E4M3) thvm_launch(true, true, k_mla_prep<true>, grid, dim3(256), (uint32_t)lds, s, *a);
-  else thvm_launch(true, true, k_mla_prep<false>, grid, dim3(256), (uint32_t)lds, s, *a);
+  const bool f8 = a->wdt == THVM_DT_FP8E4M3;
+  // MFMA wherever its 16-byte loads and stores are aligned (q rows: every
+  // head's nope part; W_uk rows hold whole 16-value pieces) and its 32-bit
+  // offsets reach the last q row
+  const bool mf = a->dn % 16 == 0 && a->dr % 8 == 0 && a->ldq % 8 == 0 &&
+                  (((uintptr_t)a->qkv | (uintptr_t)a->suk | (uintptr_t)a->qlat) & 15) == 0 &&
+                  (uint64_t)a->B * a->ldq * 2 < BUF_OOB;
+  if (mf) {
+    const dim3 grid(2 * a->B + a->H * QB * ((a->B + 15) / 16));
+    if (f8) thvm_launch(true, true, k_mla_prep_mf<true>, grid, dim3(256), 0, s, *a);
+    else thvm_launch(true, true, k_mla_prep_mf<false>, grid, dim3(256), 0, s, *a);
+  } else {
+    const dim3 grid(2 * a->B + a->H * QB * BG);
+    if (f8) thvm_launch(true, true, k_mla_prep<true>, grid, dim3(256), (uint32_t)lds, s, *a);
+    else thvm_launch(true, true, k_mla_prep<false>, grid, dim3(256), (uint32_t)lds, s, *a);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { snprintf(err, errlen, "mla_prep launch: %s", hipGetErrorString(e)); return -1; }
   return 0;
