@@ -606,6 +606,33 @@ static bool attn_mf_can(const ThvmAttnArgs *a) {
          (G & (G - 1)) == 0;
 }
 
+// One launch in which a block takes every chunk of its (row, kv head) and
+// writes the output itself, as fused = 2 picks it: no partials, and none of
+// the ~3 us that their hand-off (or a second launch) takes.  What it gives up
+// is the chunks running side by side, so the line lies at a block's work,
+// n_split G hd products a cache row; from half the CUs up in blocks the other
+// forms have nothing left to spread over, and it wins up to 16 chunks.
+// Measured on gfx950, us per launch in a graph, the form picked before -> this
+// (a full cache; at half the length it gains more):
+//   fp16 hd 64 G 1, 8 rows x 25 heads: 3 chunks 8.6 -> 5.1, 8 chunks 11.1 ->
+//   7.7, 16 chunks 16.1 -> 11.5; 12 heads: 8 chunks 7.1 -> 5.3, 9 chunks 7.1
+//   -> 6.2, but 16 chunks 7.8 -> 9.4; f32, 12 heads: 9 chunks 7.7 -> 8.0;
+//   bf16 hd 128 G 4: 3 chunks x 32 9.5 -> 9.1, 8 chunks x 256 23.1 -> 17.5,
+//   but 8 chunks x 64 12.3 -> 16.2; hd 128 G 2: 8 chunks x 32 9.4 -> 10.8.
+// The forced one-launch form (fused = 1) keeps the split of auto_cpb.
+static bool attn_whole(const ThvmAttnArgs *a) {
+  const uint32_t G = a->Hkv ? a->H / a->Hkv : 0, bh = a->B * a->Hkv;
+  if (a->fused != 2 || a->mf == 1 || (a->cpb && a->cpb < a->n_split) || (G != 1 && G != 2 && G != 4)) return false;
+  const uint64_t work = (uint64_t)a->n_split * G * a->hd;
+  if (a->n_split <= 8) return work <= 1536 || bh >= 128;
+  return G == 1 && a->n_split <= 16 && (bh >= 128 || (a->cdt != THVM_DT_FP32 && work <= 768));
+}
+
+// split and merge in one launch: asked for, or the shape's pick
+static bool attn_one_launch(const ThvmAttnArgs *a) {
+  return a->fused == 1 || (a->fused == 2 && (a->n_split <= 8 || attn_whole(a)));
+}
+
 // chunks per block of the MFMA split for cpb = 0: the grid one round of
 // blocks per CU where the rows allow (at most 256 blocks of 8 waves)
 static uint32_t attn_mf_cpb(const ThvmAttnArgs *a) {
@@ -619,15 +646,15 @@ static uint32_t attn_mf_cpb(const ThvmAttnArgs *a) {
 // wherever it applies (measured on gfx950 at the C4 head shape, split +
 // merge per launch in a graph: batch 1 10.3 against 12.3 us, batch 4 15.1
 // against 20.3, batch 16 31.5 against 38.4), except where the VALU split
-// runs as one launch by default (at most 8 chunks: the kernel boundary it
-// saves outweighs its arithmetic, C3 and C1) and in a speculative verify,
+// runs as one launch by default (at most 8 chunks, or attn_whole: the kernel
+// boundary it saves outweighs its arithmetic, C3 and C1) and in a speculative verify,
 // whose rows follow the base step's plan, passed explicitly (mf, cpb).
 extern "C" void thvm_k_attn_plan(const ThvmAttnArgs *a, uint32_t *mf, uint32_t *cpb) {
-  const bool one_launch = a->fused == 1 || (a->fused == 2 && a->n_split <= 8);
+  const bool one_launch = attn_one_launch(a);
   const bool use = a->mf == 1 || (a->mf == 0 && !a->spec && !one_launch && attn_mf_can(a));
   uint32_t c = a->cpb;
   if (c > a->n_split) c = a->n_split;
-  if (c == 0) c = use ? attn_mf_cpb(a) : thvm_k_attn_auto_cpb(a->B, a->H, a->Hkv, a->n_split, one_launch);
+  if (c == 0) c = use ? attn_mf_cpb(a) : attn_whole(a) ? a->n_split : thvm_k_attn_auto_cpb(a->B, a->H, a->Hkv, a->n_split, one_launch);
   *mf = use ? 1u : 0u;
   *cpb = c;
 }
@@ -711,7 +738,8 @@ extern "C" int thvm_k_attn_decode(const ThvmAttnArgs *a, hipStream_t s, char *er
   }
   // fused = 1: the last split block of a (row, kv head) merges in the same
   // launch; 0: a second launch merges; 2 (the shape's pick): one launch for
-  // caches of at most 8 chunks (512 rows), two above.  Measured in a graph on
+  // caches of at most 8 chunks (512 rows) and where attn_whole says so, two
+  // above.  Measured in a graph on
   // gfx950: one launch wins at short caches (C3 B=1 1.809 -> 1.767 ms, C3 B=8
   // 2.372 -> 2.285, C1 0.396 -> 0.390 ms per step), two launches at long ones
   // (C4: 11.1 against 11.9 us at L = 2051; B=16 3.50 against 3.59 ms).
@@ -724,14 +752,11 @@ extern "C" int thvm_k_attn_decode(const ThvmAttnArgs *a, hipStream_t s, char *er
                "(hd=%u G=%u)", a->hd, G);
       return -1;
     }
-    uint32_t mf = 0, cpb = 0;
-    thvm_k_attn_plan(a, &mf, &cpb);
-    if (mf) return attn_mf_launch(a, s, err, errlen);
   }
-  const bool fused = a->fused == 1 || (a->fused == 2 && a->n_split <= 8);
-  uint32_t cpb = a->cpb;
-  if (cpb > a->n_split) cpb = a->n_split;          // one block takes every chunk
-  if (cpb == 0) cpb = thvm_k_attn_auto_cpb(a->B, a->H, a->Hkv, a->n_split, fused);
+  uint32_t mf = 0, cpb = 0;
+  thvm_k_attn_plan(a, &mf, &cpb);
+  if (mf) return attn_mf_launch(a, s, err, errlen);
+  const bool fused = attn_one_launch(a);
   attn_fn f = nullptr, fm = nullptr;
   const uint32_t G = a->H / a->Hkv;
   const int at = a->cdt == THVM_DT_BF16 ? AT_BF16 : a->cdt == THVM_DT_FP16 ? AT_F16 : AT_F32;
