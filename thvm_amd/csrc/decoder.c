@@ -219,7 +219,7 @@ static int op_add(Decoder *d, const char *name, const char *prog, const u32 *arg
       prog_u32(prog, "path", 0) != 1 && prog_u32(prog, "m", 0) > 4) {
     const u32 wt = prog_u32(prog, "wt", 0), xt = prog_u32(prog, "xt", THVM_DT_BF16), k = prog_u32(prog, "k", 0);
     const u32 nrm = prog_u32(prog, "norm", 0);
-    const int mfma = (nrm == 0 || (nrm == 1 && xt == THVM_DT_BF16)) && k % 64 == 0 &&
+    const int mfma = (nrm == 0 || (nrm == 1 && xt == THVM_DT_BF16) || prog_u32(prog, "pre", 0)) && k % 64 == 0 &&
                      ((wt == THVM_DT_FP16 && xt == THVM_DT_FP16) ||
                                      (wt == THVM_DT_BF16 && xt == THVM_DT_BF16) ||
                                      (wt == THVM_DT_FP8E4M3 && (xt == THVM_DT_BF16 || xt == THVM_DT_FP16)));
@@ -497,9 +497,10 @@ static int op_attn(Decoder *d, u32 l) {
   return op_add(d, "attn", p, a, 6);
 }
 
-/* The norm feeding a GEMV: fused into the GEMV's x staging (default; above
- * 4 rows the MFMA GEMM's, which fuses RMSNorm over bf16 x), or as a separate
- * norm kernel writing xn (LayerNorm or fp16 x above 4 rows, or
+/* The norm feeding a GEMV of n rows: fused into the GEMV's x staging (above 4
+ * rows the MFMA GEMM's, which fuses RMSNorm over bf16 x), ahead of the product
+ * in the MFMA GEMM's blocks (other norms over 16-bit x up to 16 rows), or as a
+ * separate norm kernel writing xn (what is left above 4 rows, or
  * THVM_HIP_UNFUSED_NORM=1 for A/B).  Above 4 rows every projection a norm
  * feeds runs on the MFMA GEMM (dim % 64 == 0 and the dtypes are checked at
  * config time).  Writes the GEMV's input id to *gin and its norm spec
@@ -507,19 +508,26 @@ static int op_attn(Decoder *d, u32 l) {
  * caller via gargs. */
 typedef struct { int kind; u32 g, b; } NormSpec;
 
-static int fused_norms(const Decoder *d, const NormSpec *ns) {
+/* 0: a kernel of its own; 1: in the x staging; 2: ahead of the product.  Ahead,
+ * every block takes the rows' statistics (dims it holds in registers), so it is
+ * for grids of one round: 256 blocks of 2 16-row tiles (us in a graph, fp16, 8
+ * rows, norm and GEMM in two launches -> one: 4800 x 1600 9.4 -> 8.7, 2304 x 768
+ * 7.4 -> 6.9; with 4 tiles a block 16384 x 1600 17.2 -> 22.2, from spills). */
+static int fused_norms(const Decoder *d, const NormSpec *ns, u32 n) {
   const char *e = getenv("THVM_HIP_UNFUSED_NORM");
   if (e && e[0] == '1') return 0;
-  return d->rows <= 4 || (ns->kind == 1 && d->c.adtype == THVM_DT_BF16);
+  if (d->rows <= 4 || (ns->kind == 1 && d->c.adtype == THVM_DT_BF16)) return 1;
+  return d->rows <= 16 && d->c.adtype != THVM_DT_FP32 && d->c.dim <= 2048 && n <= 8192 ? 2 : 0;
 }
 
-static int emit_norm(Decoder *d, const NormSpec *ns, u32 *gin, char *nspec, size_t nlen,
+static int emit_norm(Decoder *d, const NormSpec *ns, u32 n, u32 *gin, char *nspec, size_t nlen,
                      u32 *gargs, u32 *ng) {
   const ThvmDecodeConfig *c = &d->c;
   u32 x = act(d, "x"), xn = act(d, "xn");
+  const int fuse = fused_norms(d, ns, n);
   *ng = 0;
-  if (fused_norms(d, ns)) {
-    snprintf(nspec, nlen, " norm=%d eps=%a", ns->kind, c->eps);
+  if (fuse) {
+    snprintf(nspec, nlen, " norm=%d eps=%a%s", ns->kind, c->eps, fuse == 2 ? " pre=1" : "");
     gargs[(*ng)++] = ns->g;
     if (ns->kind == 2) gargs[(*ng)++] = ns->b;
     *gin = x;
@@ -538,7 +546,7 @@ static int op_tail(Decoder *d, u32 lm_w, u32 lm_s, const NormSpec *fn) {
   const ThvmDecodeConfig *c = &d->c;
   char p[400], nsp[96];
   u32 gin, gargs[2], ng;
-  if (emit_norm(d, fn, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+  if (emit_norm(d, fn, c->vocab, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
   /* LM head -> f32 logits */
   snprintf(p, sizeof p, "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=0%s",
            d->rows, c->vocab, c->dim, c->arch == THVM_ARCH_GPT2 ? c->adtype : c->wdtype,
@@ -680,7 +688,7 @@ static int llama_ops(Decoder *d) {
     char nsp[96];
     u32 gin, gargs[2], ng;
     NormSpec n1 = {1, ga, 0};
-    if (emit_norm(d, &n1, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+    if (emit_norm(d, &n1, nqkv, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
     snprintf(p, sizeof p,
              "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=%u h=%u hkv=%u hd=%u maxseq=%u%s%s",
              B, nqkv, D, c->wdtype, adt, adt, THVM_EPI_QKV_ROPE, H, Hkv, hd, c->max_seq, nsp,
@@ -705,7 +713,7 @@ static int llama_ops(Decoder *d) {
 
     d->cur_tag = (int32_t)(2 * l + 1);
     NormSpec n2 = {1, gf, 0};
-    if (emit_norm(d, &n2, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+    if (emit_norm(d, &n2, 2 * F, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
     snprintf(p, sizeof p, "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=%u%s", B, 2 * F,
              D, c->wdtype, adt, adt, THVM_EPI_SWIGLU, nsp);
     u32 ga2[7], gn = 0;
@@ -852,7 +860,7 @@ static int build_gpt2(Decoder *d) {
     char nsp[96];
     u32 gin, gargs[2], ng;
     NormSpec n1 = {2, g1, b1};
-    if (emit_norm(d, &n1, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+    if (emit_norm(d, &n1, 3 * D, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
     snprintf(p, sizeof p,
              "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=%u bias=1 h=%u hkv=%u hd=%u maxseq=%u%s",
              B, 3 * D, D, wdt, adt, adt, THVM_EPI_QKV, H, H, hd, c->max_seq, nsp);
@@ -868,7 +876,7 @@ static int build_gpt2(Decoder *d) {
     if (op_add(d, "gemv_o", p, oa, 5)) return -1;
     d->cur_tag = (int32_t)(2 * l + 1);
     NormSpec n2 = {2, g2, b2};
-    if (emit_norm(d, &n2, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+    if (emit_norm(d, &n2, F, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
     snprintf(p, sizeof p, "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=%u bias=1%s", B,
              F, D, wdt, adt, adt, THVM_EPI_GELU, nsp);
     u32 fa[6], fn = 0;
@@ -1016,7 +1024,7 @@ static int build_dsv2(Decoder *d) {
     char nsp[96];
     u32 gin, gargs[2], ng;
     NormSpec n1 = {1, win, 0};
-    if (emit_norm(d, &n1, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+    if (emit_norm(d, &n1, nqkv, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
     snprintf(p, sizeof p, "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=0%s", B, nqkv, D,
              wdt, THVM_DT_BF16, THVM_DT_BF16, nsp);
     u32 qa[8], qn = 0;
@@ -1064,7 +1072,7 @@ static int build_dsv2(Decoder *d) {
       WM("l%u.wgu", 2 * F, D, &wgu, &sgu);
       WM("l%u.wd", D, F, &wd, &sd);
       NormSpec n2 = {1, wpost, 0};
-      if (emit_norm(d, &n2, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
+      if (emit_norm(d, &n2, 2 * F, &gin, nsp, sizeof nsp, gargs, &ng)) return -1;
       snprintf(p, sizeof p, "thvm-builtin:gemv m=%u n=%u k=%u wt=%u xt=%u yt=%u epi=%u%s", B, 2 * F,
                D, wdt, THVM_DT_BF16, THVM_DT_BF16, THVM_EPI_SWIGLU, nsp);
       u32 ga[7], gn = 0;

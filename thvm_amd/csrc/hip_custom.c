@@ -203,7 +203,7 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
          spec_u32(&sp, "path", &a.tune_path, 0, 0) || spec_u32(&sp, "spec", &a.spec, 0, 0) ||
          spec_u32(&sp, "tiled", &a.wtiled, 0, 0) || spec_u32(&sp, "clk", &a.clk_cap, 0, 0) ||
          spec_u32(&sp, "xqs", &a.xqs, 0, a.K) || spec_u32(&sp, "ws", &a.wide, 0, 0) ||
-         spec_u32(&sp, "seq", &a.seq, 0, 0));
+         spec_u32(&sp, "seq", &a.seq, 0, 0) || spec_u32(&sp, "pre", &a.pre, 0, 0));
     {
       u32 ldy0 = a.epi == THVM_EPI_SWIGLU ? a.N / 2
                : (a.epi == THVM_EPI_QKV || a.epi == THVM_EPI_QKV_ROPE) ? a.n_heads * a.head_dim

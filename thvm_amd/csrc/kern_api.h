@@ -85,6 +85,9 @@ typedef struct ThvmGemvArgs {
    * position L-1 + m % seq of sequence m / seq.  splits and vec4 are the
    * launcher's. */
   uint32_t wide, seq, splits, vec4;
+  /* MFMA GEMM, M <= 16: the norm is applied ahead of the product, rounded to
+   * xdt as the norm kernel stores it (LayerNorm, or RMSNorm over fp16 x) */
+  uint32_t pre;
   void *ws;
   uint64_t ws_bytes;
 } ThvmGemvArgs;

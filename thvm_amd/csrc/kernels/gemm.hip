@@ -31,6 +31,14 @@
 //     with the norm kernel's rnd((x * inv) * g), at a different point; bf16
 //     keeps f32's exponent range, so x*g cannot overflow where x*inv*g would
 //     not.  The batched decode step then needs no separate norm launch.
+//   * a norm ahead of the product (NM = 2, M <= 16, K <= GEMM_PRE_K: LayerNorm,
+//     or RMSNorm over fp16 x, whose products would overflow unscaled): every
+//     block takes all rows' statistics itself, two rows a wave held in
+//     registers (mean, then the squared distances from it), while its first
+//     weights are in flight, and stages rnd(((x - mean) * inv) * g + b) -- the
+//     norm kernel's value at the norm kernel's rounding.  It costs the GEMM
+//     2.2 us where the norm's own launch took 2.9 (4800 x 1600 fp16, 8 rows:
+//     9.4 -> 8.7 us for the pair).
 // MFMA operand k order: both operands give lane group g the same 8 k values
 // per instruction (k = 16g + j, then 16g + 8 + j), so the sum over k is the
 // full dot product whatever order the unit consumes them in.
@@ -40,6 +48,17 @@
 #include "epilogue.h"
 #include "mfma_ops.h"
 #include <stdio.h>
+
+// eight 16-bit values as f32
+template <int XT>
+__device__ __forceinline__ void x8(const uint4 &q, float v[8]) {
+  const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    v[2 * j] = XT == GX_BF16 ? __uint_as_float(w[j] << 16) : h2f((f16_t)(w[j] & 0xffffu));
+    v[2 * j + 1] = XT == GX_BF16 ? __uint_as_float(w[j] & 0xffff0000u) : h2f((f16_t)(w[j] >> 16));
+  }
+}
 
 #define GEMM_WAVES 8
 #define GEMM_THREADS (64 * GEMM_WAVES)
@@ -58,11 +77,14 @@
 #endif
 #define GEMM_SC(MT) (GEMM_XSTAGE / (MT))
 #define GEMM_XROW(MT) (GEMM_SC(MT) * 128 + 16)
+#define GEMM_PRE_K 2048                            // NM = 2: a row is 4 16-byte pieces a lane
 template <int WT, int XT, int MT, int NT, int U, int NM>
 __global__ __launch_bounds__(GEMM_THREADS) void k_gemm(ThvmGemvArgs a) {
   extern __shared__ float4 red[];                 // x staging, then [GEMM_WAVES][NT*MT][64]
-  __shared__ float ssw[NM ? GEMM_WAVES : 1][NM ? 64 : 1];   // per-wave sums of x^2 per x row
-  static_assert(!NM || XT == GX_BF16, "the fused norm stages bf16 x");
+  __shared__ float ssw[NM == 1 ? GEMM_WAVES : 1][NM == 1 ? 64 : 1];   // per-wave sums of x^2 per x row
+  __shared__ float2 st[NM == 2 ? 16 : 1];                   // (mean, inv) per x row
+  static_assert(NM != 1 || XT == GX_BF16, "the fused RMSNorm stages bf16 x");
+  static_assert(NM != 2 || MT == 1, "the norm ahead takes one x tile");
   constexpr int WB = WT == GW_FP8 ? 1 : 2;        // uint4 per lane per step per W tile
   constexpr int SC = GEMM_SC(MT), XROW = GEMM_XROW(MT);
   static_assert(SC % U == 0, "sub-chunks hold whole prefetch rounds");
@@ -121,7 +143,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_gemm(ThvmGemvArgs a) {
   // wave's slice (steps past s1 are staged for zero weights and must not
   // count twice), and the lane's running sums of x^2, one per staged row
   const buf_t grs = buf_rsrc(NM ? (const void *)a.norm_w : (const void *)a.x, NM ? K * 4u : 0u);
-  uint4 gv[2];
+  const buf_t brs = buf_rsrc(NM == 2 && a.norm_b ? (const void *)a.norm_b : (const void *)a.x, NM == 2 && a.norm_b ? K * 4u : 0u);
+  uint4 gv[2], bv[2];
   bool xok = false;
   float ss[NI];
 #pragma unroll
@@ -135,11 +158,28 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_gemm(ThvmGemvArgs a) {
       const uint32_t go = live && k < K ? k * 4 : BUF_OOB;
       gv[0] = buf_ld16(grs, go);
       gv[1] = buf_ld16(grs, go + 16);
+      if (NM == 2) { bv[0] = buf_ld16(brs, go); bv[1] = buf_ld16(brs, go + 16); }
       xok = live && sc0 + sl / 8 < s1;
     }
   };
   auto xstore = [&]() {
-    if (NM) {
+    if (NM == 2) {
+      const uint32_t gw[8] = {gv[0].x, gv[0].y, gv[0].z, gv[0].w, gv[1].x, gv[1].y, gv[1].z, gv[1].w};
+      const uint32_t bw[8] = {bv[0].x, bv[0].y, bv[0].z, bv[0].w, bv[1].x, bv[1].y, bv[1].z, bv[1].w};
+#pragma unroll
+      for (int i = 0; i < NI; i++) {
+        if ((uint32_t)(i * RPI) >= M) break;      // rows of padding: zeros, whose columns no one reads
+        const float2 ms = st[i * RPI + sr];
+        float v[8];
+        x8<XT>(xv[i], v);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          v[j] = ((v[j] - ms.x) * ms.y) * __uint_as_float(gw[j]) + __uint_as_float(bw[j]);
+        xv[i] = XT == GX_BF16 ? make_uint4(pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]), pk_bf16(v[4], v[5]), pk_bf16(v[6], v[7]))
+                              : make_uint4(pk_f16(v[0], v[1]), pk_f16(v[2], v[3]), pk_f16(v[4], v[5]), pk_f16(v[6], v[7]));
+      }
+    }
+    if (NM == 1) {
       const uint32_t gw[8] = {gv[0].x, gv[0].y, gv[0].z, gv[0].w, gv[1].x, gv[1].y, gv[1].z, gv[1].w};
 #pragma unroll
       for (int i = 0; i < NI; i++) {
@@ -199,10 +239,53 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_gemm(ThvmGemvArgs a) {
   // partial tiles summed, 7 drained
   pclk(a.clk, a.clk_cap, 0);
   const uint32_t nsub = (s1 - s0 + SC - 1) / SC;
+  constexpr int PC = NM == 2 ? GEMM_PRE_K / 512 : 1;
+  uint4 rv[2][PC];                                // rows wv and wv + 8: 16-byte pieces lane, lane + 64, ..
+  if (NM == 2) {
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int c = 0; c < PC; c++) {
+        const uint32_t row = wv + 8 * r, k = (lane + 64 * c) * 8;
+        rv[r][c] = buf_ld16(xrs, row < M && k < K ? (row * a.ldx + k) * 2 : BUF_OOB);
+      }
+  }
   xload(s0, true);
 #pragma unroll
   for (int u = 0; u < U; u++) load(u, s0 + u);
   pclk(a.clk, a.clk_cap, 1);
+  if (NM == 2) {                                  // pieces past K are zero: they add nothing to a sum
+    const float invK = 1.0f / (float)K;
+    float mean[2] = {0.f, 0.f}, s2[2] = {0.f, 0.f};
+    if (a.norm == 2) {
+#pragma unroll
+      for (int r = 0; r < 2; r++) {
+        float s = 0.f;
+#pragma unroll
+        for (int c = 0; c < PC; c++) {
+          float v[8];
+          x8<XT>(rv[r][c], v);
+          s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+        }
+        mean[r] = wave_sum(s) * invK;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+#pragma unroll
+      for (int c = 0; c < PC; c++) {
+        float v[8];
+        x8<XT>(rv[r][c], v);
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) s = fmaf(v[j] - mean[r], v[j] - mean[r], s);
+        s2[r] += (uint32_t)(lane + 64 * c) * 8 < K ? s : 0.f;
+      }
+      s2[r] = wave_sum(s2[r]);
+      if (lane == 0) st[wv + 8 * r] = make_float2(mean[r], 1.0f / sqrtf(s2[r] * invK + a.norm_eps));
+    }
+    __syncthreads();
+  }
   for (uint32_t c = 0; c < nsub; c++) {
     const uint32_t sb = s0 + c * SC;
     xstore();
@@ -218,7 +301,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_gemm(ThvmGemvArgs a) {
         load(u, sb + g * U + u + U);
       }
   }
-  if (NM) {   // a row's sum over the wave's slice: its 8*SC lanes, then LDS
+  if (NM == 1) {   // a row's sum over the wave's slice: its 8*SC lanes, then LDS
 #pragma unroll
     for (int i = 0; i < NI; i++) {
       float s = ss[i];
@@ -252,7 +335,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_gemm(ThvmGemvArgs a) {
       s0v += r == 0 ? q.x : q.z;
       s1v += r == 0 ? q.y : q.w;
     }
-    if (NM) {
+    if (NM == 1) {
       float t = 0.f;
 #pragma unroll
       for (int w = 0; w < GEMM_WAVES; w++) t += ssw[w][m];
@@ -278,11 +361,11 @@ static gemm_fn pick_nt(int NT) {
   switch (NT) {
     case 1: return k_gemm<WT, XT, MT, 1, U, NM>;
     case 2: return k_gemm<WT, XT, MT, 2, U, NM>;
-    case 4: return k_gemm<WT, XT, MT, 4, U4, NM>;
+    case 4: return NM < 2 ? k_gemm<WT, XT, MT, 4, U4, NM & 1> : nullptr;   // (a norm ahead spills at 4)
     // 7 or 8 tiles: one x tile and fp8 weights only (more accumulators or
     // 16-bit weight registers would spill)
-    case 7: return MT == 1 && WT == GW_FP8 ? k_gemm<GW_FP8, XT, 1, 7, 2, NM> : nullptr;
-    case 8: return MT == 1 && WT == GW_FP8 ? k_gemm<GW_FP8, XT, 1, 8, 2, NM> : nullptr;
+    case 7: return MT == 1 && NM < 2 && WT == GW_FP8 ? k_gemm<GW_FP8, XT, 1, 7, 2, NM & 1> : nullptr;
+    case 8: return MT == 1 && NM < 2 && WT == GW_FP8 ? k_gemm<GW_FP8, XT, 1, 8, 2, NM & 1> : nullptr;
     default: return nullptr;
   }
 }
@@ -300,7 +383,14 @@ static gemm_fn pick_mt(int MT, int NT) {
 // epilogue geometry); validates what only the MFMA path needs.
 extern "C" int thvm_k_gemm_mfma(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen) {
   gemm_fn f = nullptr;
-  if (a->norm && (a->norm != 1 || a->xdt != THVM_DT_BF16 || a->norm_w == nullptr)) {
+  if (a->pre) {
+    if ((a->norm != 1 && a->norm != 2) || !a->norm_w || (a->xdt != THVM_DT_BF16 && a->xdt != THVM_DT_FP16) ||
+        a->M > 16 || a->K > GEMM_PRE_K || (((uintptr_t)a->norm_w | (uintptr_t)a->norm_b) & 15)) {
+      snprintf(err, errlen, "gemm: pre=1 (a norm ahead of the product) takes norm 1 or 2 with a gain, 16-bit x, "
+               "M <= 16 and K <= %d", GEMM_PRE_K);
+      return -1;
+    }
+  } else if (a->norm && (a->norm != 1 || a->xdt != THVM_DT_BF16 || a->norm_w == nullptr)) {
     snprintf(err, errlen, "gemm: the MFMA path fuses RMSNorm with a gain over bf16 x only (norm=1, xt=bf16)");
     return -1;
   }
@@ -330,14 +420,19 @@ extern "C" int thvm_k_gemm_mfma(const ThvmGemvArgs *a, hipStream_t s, char *err,
   const uint32_t tiles = (a->N + 15u) / 16u, need = (tiles + 255u) / 256u;
   const bool wide = MT == 1 && a->wdt == THVM_DT_FP8E4M3;
   int NT = a->tune_r ? (int)a->tune_r
-         : MT == 1 ? (need <= 1 ? 1 : need == 2 ? 2 : need <= 4 || !wide ? 4 : need <= 7 ? 7 : 8)
+         : MT == 1 ? (need <= 1 ? 1 : need == 2 || a->pre ? 2 : need <= 4 || !wide ? 4 : need <= 7 ? 7 : 8)
                    : (a->N >= 16384 ? 4 : a->N <= 4096 ? 1 : 2);
   if (NT != 1 && NT != 2 && NT != 4 && !(wide && (NT == 7 || NT == 8))) {
     snprintf(err, errlen, "gemm: n tiles per block must be 1, 2 or 4 (7 or 8 with fp8 weights at M <= 16)");
     return -1;
   }
   const int xbf = a->xdt == THVM_DT_BF16, xf16 = a->xdt == THVM_DT_FP16;
-  if (a->norm) {
+  if (a->pre) {
+    if (NT > 2) { snprintf(err, errlen, "gemm: pre=1 takes 1 or 2 tiles a block"); return -1; }
+    f = a->wdt == THVM_DT_FP8E4M3 ? (xbf ? pick_nt<GW_FP8, GX_BF16, 1, 2>(NT) : pick_nt<GW_FP8, GX_F16, 1, 2>(NT))
+      : a->wdt == THVM_DT_BF16 && xbf ? pick_nt<GW_BF16, GX_BF16, 1, 2>(NT)
+      : a->wdt == THVM_DT_FP16 && xf16 ? pick_nt<GW_F16, GX_F16, 1, 2>(NT) : nullptr;
+  } else if (a->norm) {
     f = a->wdt == THVM_DT_FP8E4M3 ? pick_mt<GW_FP8, GX_BF16, 1>(MT, NT)
       : a->wdt == THVM_DT_BF16 ? pick_mt<GW_BF16, GX_BF16, 1>(MT, NT) : nullptr;
   } else if (a->wdt == THVM_DT_FP8E4M3) {

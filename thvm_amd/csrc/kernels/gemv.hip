@@ -137,12 +137,12 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   uint32_t Mk = a->M, chunks = 1;
   {
     const uint64_t xlds = (uint64_t)a->M * a->K * ((a->xdt == THVM_DT_FP32 || a->wdt == THVM_DT_FP32) ? 4 : 2);
-    const bool mfma_norm = !a->norm || (a->norm == 1 && a->xdt == THVM_DT_BF16 && a->norm_w);
+    const bool mfma_norm = !a->norm || (a->norm == 1 && a->xdt == THVM_DT_BF16 && a->norm_w) || a->pre;
     const bool mfma_types = mfma_norm && a->K % 64 == 0 &&
         ((a->wdt == THVM_DT_FP16 && a->xdt == THVM_DT_FP16) || (a->wdt == THVM_DT_BF16 && a->xdt == THVM_DT_BF16) ||
          (a->wdt == THVM_DT_FP8E4M3 && (a->xdt == THVM_DT_BF16 || a->xdt == THVM_DT_FP16)));
     const bool mfma = a->tune_path == 2 || (a->tune_path == 0 && mfma_types && (a->M > 4 || xlds > 160 * 1024));
-    if (a->wide && a->tune_path != 1 && thvm_k_gemm_wide_use(a)) {
+    if (a->wide && !a->pre && a->tune_path != 1 && thvm_k_gemm_wide_use(a)) {
       if (!mfma_types) {
         snprintf(err, errlen, "gemv: ws=1 takes 16-bit x, fp8 or the x type's weights, K %% 64 == 0 and no norm but RMSNorm over bf16");
         return -1;
@@ -150,6 +150,10 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
       return thvm_k_gemm_wide(a, s, err, errlen);
     }
     if (mfma) return thvm_k_gemm_mfma(a, s, err, errlen);
+    if (a->pre) {
+      snprintf(err, errlen, "gemv: pre=1 runs on the MFMA path only (M > 4, 16-bit x, K %% 64 == 0)");
+      return -1;
+    }
     if (a->wtiled) {
       snprintf(err, errlen, "gemv: tiled weights run on the MFMA path only (M > 4, 16-bit x, K %% 64 == 0)");
       return -1;
