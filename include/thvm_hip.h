@@ -402,9 +402,9 @@ uint32_t thvm_hip_decoder_create(const ThvmDecodeConfig *cfg, uint64_t seed);
 void     thvm_hip_decoder_destroy(uint32_t dec);
 /* Generation through the captured step (reference serve mode,
  * bench/dsv2_decode_bench.c:2749-2897): consume prompts [batch][n_prompt]
- * from position 0, one position per step (the prompt id written into the
- * device token), then decode up to max_new ids per row with the token kept
- * on the device; a row stops at `eos` (not emitted; eos < 0: never).  out
+ * from position 0, in chunks of up to 512 rows where the decoder's types and
+ * shapes allow (one position per step elsewhere), then decode up to max_new
+ * ids per row with the token kept on the device; a row stops at `eos` (not emitted; eos < 0: never).  out
  * [batch][max_new] gets the ids (-1 after a row stops), n_out[batch] their
  * counts.  Greedy or sampled as the decoder's temperature says.  The step is
  * captured on first use.  0 / -1. */

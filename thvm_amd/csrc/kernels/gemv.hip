@@ -133,7 +133,7 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   if (a->tune_path > 2) { snprintf(err, errlen, "gemv: path must be 0, 1 or 2"); return -1; }
   // row chunks: M > 4 with operands the MFMA GEMM does not take (f32 weights
   // or x, mixed 16-bit types, a fused LayerNorm or a norm over 16-bit x
-  // other than bf16) runs as M/4 chunks of 4 rows
+  // other than bf16, without pre=1) runs as M/4 chunks of 4 rows
   uint32_t Mk = a->M, chunks = 1;
   {
     const uint64_t xlds = (uint64_t)a->M * a->K * ((a->xdt == THVM_DT_FP32 || a->wdt == THVM_DT_FP32) ? 4 : 2);
