@@ -1338,10 +1338,10 @@ static int prompt_layers(Decoder *d, u32 T) {
   return 0;
 }
 
-/* Consume prompts [batch][ld], positions [0, n), leaving every buffer a step
- * reads as n steps would; with tail, the logits and the next token of the last
- * position too.  1 done, 0 not for this model or length, -1 failure. */
-int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 ld, u32 n, int tail) {
+/* Consume prompts [batch][n], leaving every buffer a step reads as n steps
+ * would, the logits and the next token of the last position included.  1 done,
+ * 0 not for this model or length, -1 failure. */
+int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 n) {
   Decoder *d = dec_get(hdl);
   if (!d) return -1;
   const ThvmDecodeConfig *c = &d->c;
@@ -1349,7 +1349,7 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 ld, u32 n, int tail) 
   if (n < 2 || !prompt_can(d) || thvm_hip_jit_is_capturing()) return 0;
   for (u32 i = 0; i < n; i++)
     for (u32 b = 0; b < B; b++) {
-      const int32_t t = prompts[(u64)b * ld + i];
+      const int32_t t = prompts[(u64)b * n + i];
       if (t < 0 || (u32)t >= c->vocab) {
         hb_set_error("decoder_generate: token %d of row %u outside [0, %u)", t, b, c->vocab);
         return -1;
@@ -1370,13 +1370,13 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 ld, u32 n, int tail) 
   for (u32 p0 = 0; p0 < n && !rc; p0 += T) {
     T = n - p0 < PROMPT_ROWS / B ? n - p0 : PROMPT_ROWS / B;
     const int32_t L = (int32_t)p0 + 1;
-    for (u32 b = 0; b < B; b++) memcpy(tok + (u64)b * T, prompts + (u64)b * ld + p0, (u64)T * 4);
+    for (u32 b = 0; b < B; b++) memcpy(tok + (u64)b * T, prompts + (u64)b * n + p0, (u64)T * 4);
     rc = thvm_hip_buf_write(tens_find(d, "p.tok"), tok, (u64)B * T * 4) ||
          thvm_hip_buf_write(tens_find(d, "len"), &L, 4) || prompt_layers(d, T);
   }
   for (u32 b = 0; b < B && !rc; b++) {
-    rc = thvm_hip_buf_write_at(tens_find(d, "hist"), (u64)b * (c->max_seq + 1) * 4, prompts + (u64)b * ld, (u64)n * 4);
-    tok[b] = prompts[(u64)b * ld + n - 1];
+    rc = thvm_hip_buf_write_at(tens_find(d, "hist"), (u64)b * (c->max_seq + 1) * 4, prompts + (u64)b * n, (u64)n * 4);
+    tok[b] = prompts[(u64)b * n + n - 1];
   }
   if (!rc) rc = thvm_hip_decoder_set_state(hdl, tok, n - 1);
   free(tok);
@@ -1386,7 +1386,7 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 ld, u32 n, int tail) 
                                   (const char *)hb_buf_ptr(tens_find(d, "p.x")) + (u64)(T - 1) * D * as,
                                   (u64)T * D * as, (u64)D * as, B, hipMemcpyDeviceToDevice, HB_STREAM);
   if (e != hipSuccess) { hb_set_error("decoder_generate: %s", hipGetErrorString(e)); return -1; }
-  for (u32 i = 0; i < d->n_ops && tail; i++)
+  for (u32 i = 0; i < d->n_ops; i++)
     if (d->ops[i].tag == -2 && run_now(d->ops[i].prog, d->ops[i].args, d->ops[i].n_args)) return -1;
   return 1;
 }

@@ -52,9 +52,9 @@ void hb_decoder_reset(void);
 void hb_loader_reset(void);
 int  hb_decoder_dims(u32 h, u32 *batch, u32 *max_seq, u32 *vocab);   /* -1: no such decoder */
 u32  hb_decoder_slot(u32 h);                                          /* its JIT slot, 0 = none */
-/* read positions [0, n) of prompts [batch][ld] in chunks (tail: with the last
- * one's logits and next token); 1 done, 0 not for this model or length, -1 */
-int  hb_decoder_prompt(u32 h, const int32_t *prompts, u32 ld, u32 n, int tail);
+/* read prompts [batch][n] in chunks, the last position's logits and next token
+ * included; 1 done, 0 not for this model or length, -1 */
+int  hb_decoder_prompt(u32 h, const int32_t *prompts, u32 n);
 u32  hb_decoder_spec_rows(u32 h);                                     /* S of its speculative step, 0 = none */
 u32  hb_decoder_spec_slot(u32 h);                                     /* that step's JIT slot, 0 = none */
 

@@ -37,25 +37,27 @@ static int gen_step(uint32_t h) {
 
 /* Generation through the speculative step (reference run_spec /
  * serve_gen_spec, bench/dsv2_decode_bench.c:2629-2745, 2798-2860): the
- * prompt's first n_prompt-1 ids go through the one-row step, the last one
- * becomes the pending id the first speculative step verifies (P = n_prompt-1);
- * each step then commits 1..S ids (hist[P+1..]), read back once per burst.
+ * prompt is read in chunks where the model allows, exactly as the plain
+ * request reads it, so the caches and the first new id, which is then the
+ * pending one, are the same bits; else its first n_prompt-1 ids go through the
+ * one-row step and the last one is the pending id (P = n_prompt-1).  Each step
+ * then commits 1..S ids (hist[P+1..]), read back once per burst.
  * A burst of n steps may advance the position by up to n*S, so it is sized
  * to keep every step's verify rows inside max_seq; when not even one fits,
  * the one-row step finishes the request. */
 static int generate_spec(uint32_t h, const int32_t *prompt, uint32_t np, uint32_t max_new,
                          int32_t eos, int32_t *out, uint32_t *n_out, u32 S, u32 max_seq) {
-  int rc = hb_decoder_prompt(h, prompt, np, np - 1, 0);
+  int rc = hb_decoder_prompt(h, prompt, np);
   if (rc < 0) return -1;
-  const u32 i0 = rc ? np - 1 : 0;
+  const u32 chunked = rc > 0;
   rc = 0;
-  for (u32 i = i0; i + 1 < np && !rc; i++) rc = thvm_hip_decoder_set_state(h, &prompt[i], i) || gen_step(h);
-  if (!rc) rc = thvm_hip_decoder_set_state(h, &prompt[np - 1], np - 1);
+  for (u32 i = 0; !chunked && i + 1 < np && !rc; i++) rc = thvm_hip_decoder_set_state(h, &prompt[i], i) || gen_step(h);
+  if (!chunked && !rc) rc = thvm_hip_decoder_set_state(h, &prompt[np - 1], np - 1);
   int32_t *hist = (int32_t *)malloc((u64)(max_seq + 1) * 4);
   if (!hist) { hb_set_error("decoder_generate: out of host memory"); return -1; }
   *n_out = 0;
   for (u32 k = 0; k < max_new; k++) out[k] = -1;
-  u32 L = np;                      /* device length: P = L-1 is the pending position */
+  u32 L = np + chunked;            /* device length: P = L-1 is the pending position */
   while (!rc) {
     /* generated ids: hist[np .. L-1] (the new pending id included) */
     const u32 have = L - np;
@@ -109,7 +111,7 @@ THVM_API int thvm_hip_decoder_generate(uint32_t h, const int32_t *prompts, uint3
   if (!tok || !hist) { free(tok); free(hist); hb_set_error("decoder_generate: out of host memory"); return -1; }
   /* prefill: position i consumes prompt id i (reference serve_prefill), in
    * chunks where the model and the length allow, else a step per position */
-  int rc = hb_decoder_prompt(h, prompts, n_prompt, n_prompt, 1);
+  int rc = hb_decoder_prompt(h, prompts, n_prompt);
   const u32 i0 = rc > 0 ? n_prompt : 0;
   if (rc > 0) rc = 0;
   for (u32 i = i0; i < n_prompt && !rc; i++) {
