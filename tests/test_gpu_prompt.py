@@ -149,6 +149,30 @@ def test_generate_continues_after_a_chunked_prompt(hip):
         dec.close()
 
 
+@pytest.mark.parametrize("new", [0, 1])
+def test_replay_after_a_chunked_prompt(hip, new):
+    """A fresh decoder's generate() leaves a step to replay, also where the
+    request ends before any step ran; without a request replay stays refused."""
+    prompt = np.random.default_rng(3).integers(0, LLAMA["vocab"], (1, 20)).astype(np.int32)
+    say("case: replay after a chunked prompt", new)
+    ids = []
+    for replay in (False, True):
+        dec = hip.Decoder(seed=11, **LLAMA)
+        try:
+            if replay:
+                with pytest.raises(hip.ThvmHipError, match="no captured step"):
+                    dec.replay(1)
+                dec.generate(prompt, new)
+                dec.replay(9)
+                assert dec.position == 20 + 9
+            else:
+                dec.generate(prompt, 10)
+            ids.append(dec.tokens(30))
+        finally:
+            dec.close()
+    assert np.array_equal(ids[0], ids[1])
+
+
 @pytest.mark.parametrize("n,new", [(2, 24), (50, 24), (50, 0), (50, 1)])
 def test_speculative_generate_after_a_chunked_prompt(hip, n, new):
     """A speculative request reads its prompt in the plain request's chunks: the

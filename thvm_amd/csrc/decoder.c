@@ -56,6 +56,7 @@ typedef struct {
   DOp *ops;
   u32 n_ops, cap_ops;
   u32 jit_slot;
+  int prompted;           /* read a prompt in chunks, so maybe before any step was captured */
   u32 n_split;
   u64 weight_bytes;       /* streamed weight + scale bytes per step */
   /* op emission: the rows of the step being built, speculative verify, and
@@ -1388,6 +1389,7 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 n) {
   if (e != hipSuccess) { hb_set_error("decoder_generate: %s", hipGetErrorString(e)); return -1; }
   for (u32 i = 0; i < d->n_ops; i++)
     if (d->ops[i].tag == -2 && run_now(d->ops[i].prog, d->ops[i].args, d->ops[i].n_args)) return -1;
+  d->prompted = 1;
   return 1;
 }
 
@@ -1467,9 +1469,11 @@ THVM_API uint32_t thvm_hip_decoder_capture(uint32_t h) {
 THVM_API int thvm_hip_decoder_replay(uint32_t h, uint32_t n) {
   Decoder *d = dec_get(h);
   if (!d) return -1;
-  if (!d->jit_slot) { hb_set_error("decoder_replay: no captured step"); return -1; }
+  if (!d->jit_slot && !d->prompted) { hb_set_error("decoder_replay: no captured step"); return -1; }
+  /* after a prompt read in chunks the step is captured here on first use (the
+   * capture runs it): a program may replay on from any generate() */
   for (u32 i = 0; i < n; i++)
-    if (thvm_hip_jit_replay(d->jit_slot)) return -1;
+    if (d->jit_slot ? thvm_hip_jit_replay(d->jit_slot) : !thvm_hip_decoder_capture(h)) return -1;
   return 0;
 }
 

@@ -136,8 +136,7 @@ THVM_API int thvm_hip_decoder_generate(uint32_t h, const int32_t *prompts, uint3
     }
     if (done_rows == B || have == max_new) break;
     const u32 burst = max_new - have < 8 ? max_new - have : 8;
-    const u32 first = hb_decoder_slot(h) ? 0 : 1;        /* the capture runs a step */
-    if ((first && gen_step(h)) || (burst > first && thvm_hip_decoder_replay(h, burst - first))) { rc = -1; break; }
+    if (thvm_hip_decoder_replay(h, burst)) { rc = -1; break; }
     have += burst;
   }
   free(done);
