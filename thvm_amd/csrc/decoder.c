@@ -210,10 +210,12 @@ static u32 tiled_copy(Decoder *d, u32 src, u32 n, u32 k, u32 wt, u32 lb) {
 
 static int op_add_raw(Decoder *d, const char *name, const char *prog, const u32 *args, u32 n);
 
-static u32 gemm_ws(Decoder *d) {
-  const u32 id = tens_find(d, "gemm.ws");
-  return id ? id : tens_new(d, "gemm.ws", THVM_DT_FP32, thvm_k_gemm_wide_ws_max());
+static u32 tens_get(Decoder *d, const char *name, u32 dt, u64 nbytes) {
+  const u32 id = tens_find(d, name);
+  return id ? id : tens_new(d, name, dt, nbytes);
 }
+
+static u32 gemm_ws(Decoder *d) { return tens_get(d, "gemm.ws", THVM_DT_FP32, thvm_k_gemm_wide_ws_max()); }
 
 static int op_add(Decoder *d, const char *name, const char *prog, const u32 *args, u32 n) {
   if (n >= 3 && d->rows > 4 && wtile_on() && strncmp(prog, "thvm-builtin:gemv ", 18) == 0 &&
@@ -1356,14 +1358,14 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 n) {
         return -1;
       }
     }
-  if (!tens_find(d, "p.x")) {            /* the chunk's workspace, kept with the decoder */
-    const u64 R = PROMPT_ROWS;
-    const u32 hq = c->n_heads * c->head_dim;
-    if (!gemm_ws(d) || !tens_new(d, "p.tok", THVM_DT_INT32, R * 4) || !tens_new(d, "p.xn", c->adtype, R * D * as) ||
-        !tens_new(d, "p.q", c->adtype, R * hq * as) || !tens_new(d, "p.att", c->adtype, R * hq * as) ||
-        !tens_new(d, "p.h", c->adtype, R * c->ffn * as) || !tens_new(d, "p.x", c->adtype, R * D * as))
-      return -1;
-  }
+  /* the chunk's workspace, kept with the decoder; no room for it: the step,
+   * which needs none */
+  const u64 R = PROMPT_ROWS;
+  const u32 hq = c->n_heads * c->head_dim;
+  if (!gemm_ws(d) || !tens_get(d, "p.tok", THVM_DT_INT32, R * 4) || !tens_get(d, "p.xn", c->adtype, R * D * as) ||
+      !tens_get(d, "p.q", c->adtype, R * hq * as) || !tens_get(d, "p.att", c->adtype, R * hq * as) ||
+      !tens_get(d, "p.h", c->adtype, R * c->ffn * as) || !tens_get(d, "p.x", c->adtype, R * D * as))
+    return 0;
   int32_t *tok = (int32_t *)malloc(PROMPT_ROWS * sizeof *tok);
   if (!tok) { hb_set_error("decoder_generate: out of host memory"); return -1; }
   int rc = 0;

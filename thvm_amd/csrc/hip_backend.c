@@ -285,6 +285,7 @@ static u32 alloc_fresh(u64 nbytes, u8 arena) {
   void *p = NULL;
   hipError_t e = hipMalloc(&p, cap_bytes);
   if (e != hipSuccess) {
+    (void)hipGetLastError();   /* a caller may go on without the block: not the next launch's error */
     slot_unuse(idx);
     hb_set_error("hipMalloc(%llu): %s", (unsigned long long)cap_bytes, hipGetErrorString(e));
     return 0;
