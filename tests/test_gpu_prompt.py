@@ -190,6 +190,4 @@ def test_speculative_generate_after_a_chunked_prompt(hip, n, new):
         finally:
             dec.close()
     assert np.array_equal(caches[0], caches[1])
-    # past the first id the verify rows repeat the one-row step, up to near ties
-    same = int(np.argmin(np.append(out[0][0] == out[1][0], False)))
-    assert same >= min(new, 8), same
+    assert np.array_equal(out[0], out[1])          # a verify row is the one-row step, bit for bit
