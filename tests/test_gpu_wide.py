@@ -182,6 +182,44 @@ def test_wide_gemm_qkv_append(hip, rope, B, T, kw):
         assert np.all(np.abs(got - want) <= bar)
 
 
+@pytest.mark.parametrize("rope", [0, 1])
+@pytest.mark.parametrize("M,ms,K", [(20, 40, 6144), (64, 40, 6144), (40, 64, 8192)])
+def test_wide_gemm_spec_append(hip, rope, M, ms, K):
+    """spec=1: the M rows are consecutive positions of one sequence, in the
+    wide GEMM as in k_gemm (the same call without ws), up to the order of the
+    sums; rows past the cache's end write nothing, and nothing is written
+    beside the one sequence's caches (views amid a larger buffer)."""
+    H, Hkv, hd, dt, pos = 4, 2, 64, DT_BF16, 9
+    N = (H + 2 * Hkv) * hd
+    say(f"case: wide gemm spec rope={rope} M={M} max_seq={ms} K={K}")
+    rng = np.random.default_rng(M + K)
+    x, w, scale, xf, wf = case(rng, DT_FP8, dt, M, N, K)
+    floor = (np.abs(xf) @ np.abs(wf).T).max()
+    ang = np.arange(ms)[:, None] * (1.0 / 10000.0 ** (np.arange(hd // 2) * 2.0 / hd))[None, :]
+    tabs = [up(hip, np.cos(ang).astype(np.float32)), up(hip, np.sin(ang).astype(np.float32))] if rope else []
+    one = Hkv * ms * hd * 2                                   # bytes of one sequence's cache
+    outs = []
+    for ws in (0, 1):
+        q, big = hip.Buffer(M * H * hd * 2), hip.Buffer(4 * M * one)
+        kc, vc = (hip.lib().thvm_hip_buf_view(big.id, o * one, one) for o in (M, 2 * M))
+        hip.builtin("gemv", [q, up(hip, x), up(hip, w), up(hip, scale), *tabs, up(hip, np.array([pos + 1], np.int32)),
+                             kc, vc, *([hip.Buffer(WS)] if ws else [])], m=M, n=N, k=K, wt=DT_FP8, xt=dt, yt=dt,
+                    epi=4 if rope else 5, h=H, hkv=Hkv, hd=hd, maxseq=ms, spec=1, **(dict(ws=1) if ws else {}))
+        raw = big.read(np.uint16).reshape(4 * M, one // 2)
+        rest = np.delete(raw, [M, 2 * M], 0)
+        assert not rest.any(), ws
+        outs.append([O.decode(a, dt).astype(np.float64) for a in (q.read(np.uint16), raw[M], raw[2 * M])])
+    live = min(M, ms - pos)
+    for a, b, rows in zip(outs[0], outs[1], (None, ms, ms)):
+        if rows:                                              # positions pos .. pos + live - 1 of each head
+            a, b = a.reshape(Hkv, ms, hd), b.reshape(Hkv, ms, hd)
+            assert b[:, pos:pos + live].any(-1).all() and not b[:, :pos].any() and not b[:, pos + live:].any()
+        # a sum that rounds the other way moves a value by an ulp (2^-7 of it at most);
+        # the rotation mixes the two of its pair, and rounds once more
+        pair = np.hypot(a[..., 0::2], a[..., 1::2]).repeat(2, -1)
+        assert np.all(np.abs(a - b) <= 2.5 * 2.0 ** -7 * pair + 2e-5 * floor)
+
+
 def test_wide_gemm_refusals(hip):
     say("case: wide gemm refusals")
     b = hip.Buffer(1 << 22)

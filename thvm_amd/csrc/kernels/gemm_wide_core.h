@@ -146,8 +146,9 @@ __device__ __forceinline__ void wide_epilogue(const ThvmGemvArgs &a, const uint3
       if (pos < 0 || (uint32_t)pos >= a.max_seq) break;
       const bool rope = a.epi == THVM_EPI_QKV_ROPE;
       float2 cs[NT][MT], sn[NT][MT];
-      // row m is position pos + m % T of sequence m / T (T rows a sequence)
-      const uint32_t T = a.seq ? a.seq : 1u;
+      // row m is position pos + m % T of sequence m / T (T rows a sequence; a
+      // speculative verify's rows are all one sequence's)
+      const uint32_t T = a.spec ? M : a.seq ? a.seq : 1u;
       WIDE_EACH(
         const uint32_t pm = (uint32_t)pos + m % T;
         const bool rot = rope && ok && n < Hq + Hk && pm < a.max_seq;
