@@ -233,3 +233,21 @@ def test_wide_gemm_refusals(hip):
     with pytest.raises(hip.ThvmHipError, match="rows a sequence"):
         hip.builtin("gemv", [b, b, b, b, b, b, b], m=70, n=256, k=256, wt=DT_BF16, xt=DT_BF16, yt=DT_BF16,
                     epi=5, h=2, hkv=1, hd=64, maxseq=8, ws=1, seq=33)
+
+
+@pytest.mark.parametrize("m,extra", [(2, dict(path=1)), (4, dict(path=1)), (6, dict(pre=1, norm=2)), (16, dict(pre=1, norm=2)),
+                                     (4, dict(spec=1)), (70, dict(spec=1)), (6, None)])
+def test_wide_gemm_seq_refusals(hip, m, extra):
+    """seq= on a QKV call that another kernel would run (one position a row),
+    or beside spec, is refused before anything is launched: the caches hold
+    m / seq sequences only."""
+    say(f"case: wide gemm seq refusal m={m} {extra}")
+    H, Hkv, hd, ms, K, dt = 2, 1, 64, 16, 256, DT_BF16
+    N = (H + 2 * Hkv) * hd
+    q, x, w = hip.Buffer(m * H * hd * 2), hip.Buffer(m * K * 2), hip.Buffer(N * K * 2)
+    norm = [hip.Buffer(K * 4), hip.Buffer(K * 4)] if extra and extra.get("norm") else []
+    kc, vc = (hip.Buffer(m // 2 * Hkv * ms * hd * 2) for _ in range(2))
+    tail = [hip.Buffer(4), kc, vc] + ([hip.Buffer(WS)] if extra is not None else [])
+    with pytest.raises(hip.ThvmHipError, match="rows a sequence"):
+        hip.builtin("gemv", [q, x, w, *norm, *tail], m=m, n=N, k=K, wt=dt, xt=dt, yt=dt, epi=5, h=H, hkv=Hkv, hd=hd,
+                    maxseq=ms, seq=2, **(dict(ws=1, **extra) if extra is not None else {}))

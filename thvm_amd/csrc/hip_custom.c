@@ -234,8 +234,11 @@ int hb_builtin_launch(const char *program, const u32 *ids, u32 n, int check_only
       a.rope_sin = (const float *)arg(&c, slot++, (u64)a.max_seq * (a.head_dim / 2) * 4);
     }
     if (qkv) {
-      if (a.seq && (a.spec || !a.wide || a.M % a.seq)) {
-        hb_set_error("builtin gemv: seq=%u rows a sequence must divide m=%u, with ws=1 and without spec", a.seq, a.M);
+      /* (the caches are sized by seq: only calls the wide GEMM runs, which is
+       * the one kernel that reads it, may carry it) */
+      if (a.seq && (a.spec || !a.wide || a.pre || a.tune_path == 1 || a.M % a.seq)) {
+        hb_set_error("builtin gemv: seq=%u rows a sequence must divide m=%u, with ws=1 and without spec, pre or path=1",
+                     a.seq, a.M);
         return -1;
       }
       u64 cb = (u64)(a.spec ? 1 : a.seq ? a.M / a.seq : a.M) * a.n_kv_heads * a.max_seq * a.head_dim * ysz;

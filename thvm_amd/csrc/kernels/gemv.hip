@@ -149,6 +149,10 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
       }
       return thvm_k_gemm_wide(a, s, err, errlen);
     }
+    if (a->seq && pairs && a->epi != THVM_EPI_SWIGLU) {   // the other kernels append one position a row
+      snprintf(err, errlen, "gemv: seq=%u needs the wide GEMM (ws=1, no pre, path not 1)", a->seq);
+      return -1;
+    }
     if (mfma) return thvm_k_gemm_mfma(a, s, err, errlen);
     if (a->pre) {
       snprintf(err, errlen, "gemv: pre=1 runs on the MFMA path only (M > 4, 16-bit x, K %% 64 == 0)");
