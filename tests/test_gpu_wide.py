@@ -251,3 +251,13 @@ def test_wide_gemm_seq_refusals(hip, m, extra):
     with pytest.raises(hip.ThvmHipError, match="rows a sequence"):
         hip.builtin("gemv", [q, x, w, *norm, *tail], m=m, n=N, k=K, wt=dt, xt=dt, yt=dt, epi=5, h=H, hkv=Hkv, hd=hd,
                     maxseq=ms, seq=2, **(dict(ws=1, **extra) if extra is not None else {}))
+
+
+def test_wide_gemm_empty_and_huge_shapes_refused(hip):
+    """No columns or rows, and counts whose tile arithmetic would leave 32 bits,
+    are errors (the workspace is sized before the launcher's range checks)."""
+    say("case: wide gemm empty and huge shapes")
+    b = hip.Buffer(1 << 16)
+    for m, n, k in ((65, 0, 64), (0, 64, 64), (65, 64, 0), (2 ** 32 - 1, 64, 64), (65, 2 ** 32 - 1, 64), (2 ** 32 - 1, 2 ** 32 - 1, 64)):
+        with pytest.raises(hip.ThvmHipError):
+            hip.builtin("gemv", [b, b, b, b], m=m, n=n, k=k, wt=DT_BF16, xt=DT_BF16, yt=DT_BF16, ws=1)

@@ -44,9 +44,12 @@ extern "C" int thvm_k_gemm_wide_use(const ThvmGemvArgs *a) {
 //   * splits fill the last round only (blocks * splits <= 256): a split costs
 //     its hand-off (~4 chunks) and a read of its tile (~1 chunk), and a block
 //     runs its chunks in fours.
+// (asked for by the builtin's argument checks too, before the launcher's: in 64
+// bits, and with no rows or columns one empty block)
+static uint64_t tiles_of(uint32_t n, uint32_t t) { return ((uint64_t)n + t - 1) / t; }
 static void wide_plan(const ThvmGemvArgs *a, int *MT, int *NT, uint32_t *SP) {
   *MT = a->M <= 32 ? 2 : 4;
-  const uint32_t mt = (a->M + 16u * *MT - 1) / (16u * *MT), g64 = (a->N + 63) / 64;
+  const uint64_t mt = tiles_of(a->M, 16u * *MT), g64 = tiles_of(a->N, 64);
   const uint32_t CH = (a->K / 64 + GW_KG - 1) / GW_KG;
   static const float chunk[3] = {0.40f, 0.56f, 1.04f};
   float best = 0.f;
@@ -55,10 +58,11 @@ static void wide_plan(const ThvmGemvArgs *a, int *MT, int *NT, uint32_t *SP) {
   for (int i = 0; i < 3; i++) {
     const int nt = 1 << i;
     if (a->tune_r ? (int)a->tune_r != nt : mt == 1 && nt != (g64 <= 256 ? 1 : g64 <= 512 ? 2 : 4)) continue;
-    const uint32_t blocks = (g64 + nt - 1) / nt * mt;
-    const uint32_t smax = a->tune_blocks ? a->tune_blocks : blocks >= 256 ? 1 : 256 / blocks < 8 ? 256 / blocks : 8;
-    for (uint32_t sp = a->tune_blocks ? smax : 1; sp <= smax && (sp == 1 || 4 * sp <= CH); sp++) {
-      const uint64_t per = ((CH + sp - 1) / sp + 3) / 4 * 4, rounds = ((uint64_t)blocks * sp + 255) / 256;
+    const uint64_t blocks = (g64 + nt - 1) / nt * mt;
+    const uint32_t smax = a->tune_blocks ? a->tune_blocks
+                        : blocks == 0 || blocks >= 256 ? 1 : 256 / blocks < 8 ? (uint32_t)(256 / blocks) : 8;
+    for (uint32_t sp = a->tune_blocks ? smax : 1; sp <= smax && (sp == 1 || 4ull * sp <= CH); sp++) {
+      const uint64_t per = ((CH + sp - 1) / sp + 3) / 4 * 4, rounds = (blocks * sp + 255) / 256;
       const float t = chunk[i] * (float)(rounds * per) + (sp > 1 ? 0.40f * (float)(4 + sp) : 0.f);
       if (best == 0.f || t < best) { best = t; *NT = nt; *SP = sp; }
     }
@@ -72,7 +76,7 @@ extern "C" uint64_t thvm_k_gemm_wide_ws(const ThvmGemvArgs *a) {
   if (!thvm_k_gemm_wide_use(a)) return 0;
   wide_plan(a, &MT, &NT, &SP);
   if (SP <= 1) return 0;
-  const uint64_t tiles = (uint64_t)((a->N + 64u * NT - 1) / (64u * NT)) * ((a->M + 16u * MT - 1) / (16u * MT));
+  const uint64_t tiles = tiles_of(a->N, 64u * NT) * tiles_of(a->M, 16u * MT);
   return GW_CTR_BYTES + tiles * SP * (GW_NWAVES * NT * MT * 1024ull + 16ull * MT * 4);
 }
 
@@ -103,7 +107,7 @@ extern "C" int thvm_k_gemm_wide(const ThvmGemvArgs *a, hipStream_t s, char *err,
   wide_plan(a, &MT, &NT, &SP);
   ThvmGemvArgs k = *a;
   k.splits = SP;
-  if (SP > 1 && (uint64_t)((a->N + 64u * NT - 1) / (64u * NT)) * ((a->M + 16u * MT - 1) / (16u * MT)) > GW_CTR_BYTES / 4) {
+  if (SP > 1 && tiles_of(a->N, 64u * NT) * tiles_of(a->M, 16u * MT) > GW_CTR_BYTES / 4) {
     snprintf(err, errlen, "gemm_wide: %u splits of more than %u tiles", SP, GW_CTR_BYTES / 4);
     return -1;
   }
@@ -132,8 +136,7 @@ extern "C" int thvm_k_gemm_wide(const ThvmGemvArgs *a, hipStream_t s, char *err,
     snprintf(err, errlen, "gemm_wide: seq needs aligned rows of four (the scalar epilogue has one position per row)");
     return -1;
   }
-  const uint32_t mt = (a->M + 16u * MT - 1) / (16u * MT), nt = (a->N + 64u * NT - 1) / (64u * NT);
-  const uint64_t total = (uint64_t)mt * nt * SP, grid = (total + 7) / 8 * 8;
+  const uint64_t total = tiles_of(a->M, 16u * MT) * tiles_of(a->N, 64u * NT) * SP, grid = (total + 7) / 8 * 8;
   if (grid > 0x7fffffffull) { snprintf(err, errlen, "gemm_wide: grid too large"); return -1; }
   const uint32_t xlds = 2u * 16u * MT * GW_XROW, elds = (uint32_t)GW_NWAVES * NT * MT * 1024u;
   const uint32_t lds = xlds > elds ? xlds : elds;
