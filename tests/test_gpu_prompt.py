@@ -191,3 +191,21 @@ def test_speculative_generate_after_a_chunked_prompt(hip, n, new):
             dec.close()
     assert np.array_equal(caches[0], caches[1])
     assert np.array_equal(out[0], out[1])          # a verify row is the one-row step, bit for bit
+
+
+@pytest.mark.parametrize("n", [3, 4, 5])
+def test_prompt_over_a_long_ffn_row(hip, n):
+    """ffn = 20480: four positions' rows of the down projection fill the GEMV's
+    LDS to the byte, so its chunk of four ids runs on the MFMA GEMM."""
+    cfg = dict(LLAMA, n_layers=1, dim=128, n_heads=2, n_kv_heads=1, ffn=20480, max_seq=64, wdtype=DT_BF16)
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], (1, n)).astype(np.int32)
+    say("case: prompt over a long ffn row", n)
+    wc, wl, _, _ = stepped(hip, cfg, prompt)
+    dec = hip.Decoder(seed=11, **cfg)
+    try:
+        dec.generate(prompt, 1)
+        gc, gl, _, gp = state(dec, cfg, n)
+    finally:
+        dec.close()
+    # (the bar of test_generate_prompt_equals_steps for bf16)
+    assert gp == n and rel(gl, wl) <= 2.5e-2 and all(rel(gc[k], wc[k]) <= 2.5e-2 for k in wc)

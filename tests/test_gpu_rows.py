@@ -48,3 +48,25 @@ def test_gemv_rows_equal_one_row(hip, wdt, xdt, N, K, norm):
         got = y.read(np.uint32).reshape(M, N)
         for r in range(M):
             assert np.array_equal(got[r], one[r]), (M, r)
+
+
+@pytest.mark.parametrize("wdt,xdt", [(DT_FP8, DT_BF16), (DT_F16, DT_F16)])
+@pytest.mark.parametrize("M,K", [(4, 20416), (4, 20480), (4, 20544), (2, 40960), (1, 81920)])
+def test_gemv_rows_at_the_lds_limit(hip, wdt, xdt, M, K):
+    """Rows that just do not fit the GEMV's LDS (160 KiB with its reserve: M K 2
+    = 163840 bytes exactly, and a step to each side) take the MFMA GEMM."""
+    N = 48
+    print(f"case: gemv rows at the LDS limit wdt={wdt} M={M} K={K}", flush=True)
+    rng = np.random.default_rng(M + K)
+    x = O.encode(rng.standard_normal((M, K)).astype(np.float32), xdt)
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    sc = (np.abs(w).max(1) / 448).astype(np.float32) if wdt == DT_FP8 else None
+    ws = O.encode(w / sc[:, None] if sc is not None else w, wdt)
+    wf = O.decode(ws, wdt).astype(np.float64) * (sc[:, None] if sc is not None else 1.0)
+    xf = O.decode(x, xdt).astype(np.float64)
+    y = hip.Buffer(M * N * 4)
+    hip.builtin("gemv", [y, up(hip, x), up(hip, ws), *([up(hip, sc)] if sc is not None else [])], m=M, n=N, k=K, wt=wdt,
+                xt=xdt, yt=DT_F32)
+    got = y.read(np.float32).reshape(M, N)
+    # f32 sums of K products in any order: well inside 2^-24 sqrt(K) of the absolute sum
+    assert np.all(np.abs(got - xf @ wf.T) <= 1e-5 * (np.abs(xf) @ np.abs(wf).T))

@@ -48,6 +48,15 @@ static int act_ok(uint32_t dt) {
   return dt == THVM_DT_FP32 || dt == THVM_DT_FP16 || dt == THVM_DT_BF16;
 }
 
+// LDS of the GEMV at M x rows: the staged rows, then a fused norm's partial sums
+// (summed x: a spare word after the row).  One bound for the path choice and for
+// the launch, so that an x too long for the GEMV always reaches the MFMA GEMM.
+#define GEMV_LDS_MAX (160u * 1024u - GEMV_MAX_WAVES * 4u)
+static uint64_t gemv_lds(const ThvmGemvArgs *a, uint32_t M) {
+  const uint64_t rows = (uint64_t)M * a->K * (a->xdt == THVM_DT_FP32 || a->wdt == THVM_DT_FP32 ? 4 : 2);
+  return rows + (a->norm == 3 ? 16u : a->norm ? M * GEMV_MAX_WAVES * 4u : 0u);
+}
+
 extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen) {
   int wsz = dt_size(a->wdt);
   if (wsz == 0 || !act_ok(a->xdt) || !act_ok(a->ydt)) {
@@ -136,12 +145,12 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   // other than bf16, without pre=1) runs as M/4 chunks of 4 rows
   uint32_t Mk = a->M, chunks = 1;
   {
-    const uint64_t xlds = (uint64_t)a->M * a->K * ((a->xdt == THVM_DT_FP32 || a->wdt == THVM_DT_FP32) ? 4 : 2);
+    const uint64_t xlds = gemv_lds(a, a->M);
     const bool mfma_norm = !a->norm || (a->norm == 1 && a->xdt == THVM_DT_BF16 && a->norm_w) || a->pre;
     const bool mfma_types = mfma_norm && a->K % 64 == 0 &&
         ((a->wdt == THVM_DT_FP16 && a->xdt == THVM_DT_FP16) || (a->wdt == THVM_DT_BF16 && a->xdt == THVM_DT_BF16) ||
          (a->wdt == THVM_DT_FP8E4M3 && (a->xdt == THVM_DT_BF16 || a->xdt == THVM_DT_FP16)));
-    const bool mfma = a->tune_path == 2 || (a->tune_path == 0 && mfma_types && (a->M > 4 || xlds > 160 * 1024));
+    const bool mfma = a->tune_path == 2 || (a->tune_path == 0 && mfma_types && (a->M > 4 || xlds > GEMV_LDS_MAX));
     if (a->wide && !a->pre && a->tune_path != 1 && thvm_k_gemm_wide_use(a)) {
       if (!mfma_types) {
         snprintf(err, errlen, "gemv: ws=1 takes 16-bit x, fp8 or the x type's weights, K %% 64 == 0 and no norm but RMSNorm over bf16");
@@ -213,15 +222,12 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   // 13.9 against 14.4); 8 would leave half the lanes idle on 256-chunk rows
   int U = a->tune_u ? (int)a->tune_u : 4;
   if (U != 4 && U != 8) { snprintf(err, errlen, "gemv: u must be 4 or 8"); return -1; }
-  uint32_t xsz = (a->xdt == THVM_DT_FP32 || a->wdt == THVM_DT_FP32) ? 4 : 2;
-  uint64_t lds = (uint64_t)Mk * a->K * xsz + (xsum ? 16 : 0);   // (summed x: a spare word after the row)
-  const uint64_t red = a->norm && !xsum ? (uint64_t)Mk * GEMV_MAX_WAVES * 4 : 0;   // the norm's partial sums
-  if (lds + (red ? red : GEMV_MAX_WAVES * 4) > 160 * 1024) {
+  const uint64_t lds = gemv_lds(a, Mk);
+  if (lds > GEMV_LDS_MAX) {
     snprintf(err, errlen, "gemv: M*K=%llu x elements exceed LDS (use the MFMA GEMM)",
              (unsigned long long)Mk * a->K);
     return -1;
   }
-  lds += red;
   gemv_fn f = nullptr;
   switch (a->wdt) {
     case THVM_DT_FP32: f = pick_x<WT_F32>(a->xdt, Mk, R, U); break;
