@@ -209,3 +209,59 @@ def test_prompt_over_a_long_ffn_row(hip, n):
         dec.close()
     # (the bar of test_generate_prompt_equals_steps for bf16)
     assert gp == n and rel(gl, wl) <= 2.5e-2 and all(rel(gc[k], wc[k]) <= 2.5e-2 for k in wc)
+
+
+def test_generate_after_a_pool_rollback(hip):
+    """The chunk workspace, made inside the first request, outlives a rollback
+    to a watermark taken before that request, and the same ids come back."""
+    cfg = dict(LLAMA, batch=2)
+    prompt = np.random.default_rng(7).integers(0, cfg["vocab"], (2, 40)).astype(np.int32)
+    say("case: generate, pool rollback, generate")
+    L = hip.lib()
+    dec = hip.Decoder(seed=11, **cfg)
+    try:
+        wm = L.thvm_hip_buf_pool_begin()
+        first, _ = dec.generate(prompt, 6)
+        L.thvm_hip_buf_pool_rollback_with_preserve(wm)
+        L.thvm_hip_buf_clear_preserved(wm)
+        again, _ = dec.generate(prompt, 6)
+        assert np.array_equal(first, again)
+    finally:
+        dec.close()
+
+
+_SWEPT_CHILD = """
+import sys
+sys.path[:0] = [{root!r}, {tests!r}]
+import numpy as np
+import thvm_amd
+import test_gpu_prompt as T
+thvm_amd.init()
+prompt = np.random.default_rng(8).integers(0, T.LLAMA["vocab"], (1, 40)).astype(np.int32)
+dec = thvm_amd.Decoder(seed=11, **T.LLAMA)
+want, _ = dec.generate(prompt, 6)
+dec.close()
+dec = thvm_amd.Decoder(seed=11, **T.LLAMA)
+dec.generate(prompt, 1)                        # ends before any step is captured
+thvm_amd.lib().thvm_hip_buf_free_unpreserved_all()
+got, _ = dec.generate(prompt, 6)
+assert np.array_equal(got, want)
+dec.close()
+thvm_amd.shutdown()
+print("swept child ok", flush=True)
+"""
+
+
+def test_generate_holds_the_step_against_a_sweep(hip):
+    """A request that ends with its prompt holds the step's buffers as one that
+    captured the step does: the table-wide sweep leaves the decoder whole (in a
+    process of its own, the sweep would take other tests' buffers)."""
+    import subprocess
+    import sys
+    from pathlib import Path
+    root = Path(__file__).resolve().parents[1]
+    say("case: generate, table-wide sweep, generate (child process)")
+    r = subprocess.run([sys.executable, "-c", _SWEPT_CHILD.format(root=str(root), tests=str(root / "tests"))],
+                       capture_output=True, text=True, timeout=100)
+    say(r.stdout[-2000:], r.stderr[-2000:])
+    assert r.returncode == 0 and "swept child ok" in r.stdout

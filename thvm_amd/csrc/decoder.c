@@ -1359,13 +1359,19 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 n) {
       }
     }
   /* the chunk's workspace, kept with the decoder; no room for it: the step,
-   * which needs none */
+   * which needs none.  Made inside a request, it is held as a captured step's
+   * buffers are: a program's pool rollback or sweep must not take it */
   const u64 R = PROMPT_ROWS;
   const u32 hq = c->n_heads * c->head_dim;
-  if (!gemm_ws(d) || !tens_get(d, "p.tok", THVM_DT_INT32, R * 4) || !tens_get(d, "p.xn", c->adtype, R * D * as) ||
-      !tens_get(d, "p.q", c->adtype, R * hq * as) || !tens_get(d, "p.att", c->adtype, R * hq * as) ||
-      !tens_get(d, "p.h", c->adtype, R * c->ffn * as) || !tens_get(d, "p.x", c->adtype, R * D * as))
-    return 0;
+  const u32 work[7] = {gemm_ws(d), tens_get(d, "p.tok", THVM_DT_INT32, R * 4), tens_get(d, "p.xn", c->adtype, R * D * as),
+                       tens_get(d, "p.q", c->adtype, R * hq * as), tens_get(d, "p.att", c->adtype, R * hq * as),
+                       tens_get(d, "p.h", c->adtype, R * c->ffn * as), tens_get(d, "p.x", c->adtype, R * D * as)};
+  int room = 1;
+  for (u32 i = 0; i < 7; i++) {
+    if (work[i]) thvm_hip_buf_jit_pin(work[i]);
+    else room = 0;
+  }
+  if (!room) return 0;
   int32_t *tok = (int32_t *)malloc(PROMPT_ROWS * sizeof *tok);
   if (!tok) { hb_set_error("decoder_generate: out of host memory"); return -1; }
   int rc = 0;
@@ -1391,6 +1397,9 @@ int hb_decoder_prompt(u32 hdl, const int32_t *prompts, u32 n) {
   if (e != hipSuccess) { hb_set_error("decoder_generate: %s", hipGetErrorString(e)); return -1; }
   for (u32 i = 0; i < d->n_ops; i++)
     if (d->ops[i].tag == -2 && run_now(d->ops[i].prog, d->ops[i].args, d->ops[i].n_args)) return -1;
+  /* and the step's buffers, as its capture on the first id would hold them */
+  for (u32 i = 0; i < d->n_ops && !d->prompted; i++)
+    for (u32 k = 0; k < d->ops[i].n_args; k++) thvm_hip_buf_jit_pin(d->ops[i].args[k]);
   d->prompted = 1;
   return 1;
 }
