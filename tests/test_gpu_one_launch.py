@@ -85,3 +85,19 @@ def test_argmax_bump_refusals(hip):
     for kw in (dict(bump=1), dict(bump=1, hist=1, hstride=4, temp=0.5)):
         with pytest.raises(hip.ThvmHipError, match="bump"):
             hip.builtin("argmax", [tok, lg, pv, pi, hist, ln], b=1, v=64, nb=8, **kw)
+
+
+@pytest.mark.parametrize("bump", [0, 1])
+@pytest.mark.parametrize("B", [17, 64, 70, 1000])
+def test_argmax_over_many_rows(hip, B, bump):
+    """Each row a block of its own, or (bump) one block whose waves take several."""
+    say(f"case: argmax rows B={B} bump={bump}")
+    V, nb, stride, L = 300, 7, 12, 5
+    lg = np.random.default_rng(B).standard_normal((B, V)).astype(np.float32)
+    lg[:, 250] = lg[:, 31] = 9.0                        # ties: the lowest index
+    tok, pv, pi, hist = (hip.Buffer(n) for n in (B * 4, B * nb * 4, B * nb * 4, B * stride * 4))
+    ln = up(hip, np.array([L], np.int32))
+    hip.builtin("argmax", [tok, up(hip, lg), pv, pi, hist, ln], b=B, v=V, nb=nb, hist=1, hstride=stride, bump=bump)
+    assert np.all(tok.read(np.int32) == 31)
+    h = hist.read(np.int32).reshape(B, stride)
+    assert np.all(h[:, L] == 31) and not np.delete(h, L, 1).any() and ln.read(np.int32)[0] == L + bump

@@ -367,15 +367,18 @@ __global__ __launch_bounds__(256) void k_argmax_part(ThvmArgmaxArgs a) {
   a.pi[b * a.nb + blk] = bi;
 }
 
-// One block, a wave per batch row: lanes scan the block partials, then a wave
-// reduction keeps (max value, lowest index).  bump: the block also advances the
-// length once every row has written its id, in place of a launch of its own
-// (1.6 us of a graph's step for one add).
+// A wave per batch row: lanes scan the block partials, then a wave reduction
+// keeps (max value, lowest index).  bump: one block takes every row and also
+// advances the length once each has written its id, in place of a launch of its
+// own (1.6 us of a graph's step for one add; still so at 60 rows of 128256
+// logits, where its waves take four rows each: 20.0 us against 21.1).  Without
+// bump each row is a block of one wave (1000 rows of 1000 logits: 14 us, in one
+// block 44).
 #define AM_FIN_WAVES 16
 __global__ __launch_bounds__(64 * AM_FIN_WAVES) void k_argmax_fin(ThvmArgmaxArgs a) {
   const int lane = lane_id();
   const int32_t L = a.len ? a.len[0] : 0;
-  for (uint32_t b = threadIdx.x >> 6; b < a.B; b += blockDim.x >> 6) {
+  for (uint32_t b = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); b < a.B; b += gridDim.x * (blockDim.x >> 6)) {
     float bv = -INFINITY;
     int32_t bi = 0x7fffffff;
     for (uint32_t k = lane; k < a.nb; k += 64) {
@@ -569,7 +572,8 @@ extern "C" int thvm_k_argmax(const ThvmArgmaxArgs *a, hipStream_t s, char *err, 
     return 0;
   }
   thvm_launch(true, false, k_argmax_part, dim3(a->nb, a->B), dim3(256), 0, s, *a);
-  thvm_launch(false, true, k_argmax_fin, dim3(1), dim3(64 * (a->B < AM_FIN_WAVES ? a->B : AM_FIN_WAVES)), 0, s, *a);
+  const uint32_t waves = !a->bump ? 1u : a->B < AM_FIN_WAVES ? a->B : AM_FIN_WAVES;
+  thvm_launch(false, true, k_argmax_fin, dim3(a->bump ? 1u : a->B), dim3(64 * waves), 0, s, *a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { snprintf(err, errlen, "argmax launch: %s", hipGetErrorString(e)); return -1; }
   return 0;
