@@ -265,3 +265,29 @@ def test_generate_holds_the_step_against_a_sweep(hip):
                        capture_output=True, text=True, timeout=100)
     say(r.stdout[-2000:], r.stderr[-2000:])
     assert r.returncode == 0 and "swept child ok" in r.stdout
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(8, 4, 64), (3, 3, 128)])
+def test_attn_prompt_keeps_p_in_f32(hip, H, Hkv, hd):
+    """Over hundreds of near-equal probabilities an output is the nearest bf16 of
+    the float64 result except where that lies within the f32 sums' error of a
+    midpoint: about c 2^-24 / 2^-8 of the values for an error of c f32 ulps (4 of
+    them give 2.5e-4; p cut to 16 bits gave 2e-3)."""
+    T, ms, dt = 500, 512, DT_BF16
+    say(f"case: attn_prompt p in f32 H={H} hd={hd}")
+    rng = np.random.default_rng(hd)
+    q = O.encode((0.2 * rng.standard_normal((1, T, H, hd))).astype(np.float32), dt)
+    k, v = (O.encode(rng.standard_normal((1, Hkv, ms, hd)).astype(np.float32), dt) for _ in range(2))
+    out, scale = hip.Buffer(T * H * hd * 2), float(np.float32(1 / np.sqrt(hd)))
+    hip.builtin("attn_prompt", [out, up(hip, q), up(hip, k), up(hip, v), up(hip, np.array([1], np.int32))],
+                b=1, t=T, h=H, hkv=Hkv, hd=hd, maxseq=ms, dt=dt, scale=scale)
+    got = out.read(np.uint16).reshape(T, H, hd)
+    qf, kf, vf = (O.decode(a, dt).astype(np.float64)[0] for a in (q, k, v))
+    off = 0
+    for h in range(H):
+        s = qf[:, h] @ kf[h * Hkv // H].T * scale
+        s = np.where(np.arange(ms)[None] <= np.arange(T)[:, None], s, -np.inf)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = (p / p.sum(-1, keepdims=True)) @ vf[h * Hkv // H]
+        off += (O.encode(want.astype(np.float32), dt) != got[:, h]).sum()
+    assert off <= 5e-4 * got.size, off / got.size

@@ -6,9 +6,12 @@
 // once per position.
 //
 // Here the 16 columns of the MFMA tiles are 16 positions of one head, where the
-// decode split has the query heads there; operand layouts, the log2-domain
-// online softmax and p as 16-bit hi + lo pairs (so p keeps ~16 significant
-// bits) are those of k_attn_mf:
+// decode split has the query heads there; operand layouts and the log2-domain
+// online softmax are those of k_attn_mf.  p keeps the 24 bits it has in the
+// one-launch decode form (f32 there), as a sum of 16-bit terms, each the
+// rounding of what the ones before leave: three in bf16 (8 bits each), two in
+// fp16 (11 each, p scaled by 2^14 so that the second stays out of fp16's
+// subnormals; the scale cancels in acc / l):
 //   * a block is 16 positions x GH heads of one kv head (GH = 2 where G is
 //     even: each K / V tile loaded serves both), 4 waves, the cache's 16-row
 //     tiles round-robin over the waves with the next one in flight;
@@ -30,7 +33,8 @@ template <int HD, int AT, int GH>
 __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
   static_assert(AT == AT_BF16 || AT == AT_F16, "16-bit caches");
   constexpr int XT = AT == AT_BF16 ? GX_BF16 : GX_F16;
-  constexpr int KS = HD / 32, NC = HD / 8;
+  constexpr int KS = HD / 32, NC = HD / 8, PT = AT == AT_BF16 ? 3 : 2;   // PT: 16-bit terms of p
+  constexpr float PS = AT == AT_BF16 ? 1.0f : 16384.0f;
   extern __shared__ __align__(16) float apl[];
   float(*const wacc)[GH * 16][HD + 4] = (float(*)[GH * 16][HD + 4])apl;      // [wave][head, position][d]
   __shared__ float wm[AP_WAVES][GH * 16], wl[AP_WAVES][GH * 16];
@@ -78,7 +82,7 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
   }
   auto tile = [&](int buf, int t) {
     const int32_t rb = 16 * t + 4 * lg;
-    uint32_t ph[GH][2], pl[GH][2];
+    uint32_t pt[GH][PT][2];
 #pragma unroll
     for (int g = 0; g < GH; g++) {
       f32x4_t sc = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -94,7 +98,7 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
       const float f = m[g] == -INFINITY ? 0.0f : fexp2(m[g] - mn);
       float p[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) p[i] = sv[i] == -INFINITY ? 0.0f : fexp2(sv[i] - mn);
+      for (int i = 0; i < 4; i++) p[i] = sv[i] == -INFINITY ? 0.0f : fexp2(sv[i] - mn) * PS;
       l[g] = l[g] * f + ((p[0] + p[1]) + (p[2] + p[3]));
       m[g] = mn;
       if (__builtin_amdgcn_ballot_w64(f != 1.0f)) {
@@ -103,16 +107,15 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; i++) acc[g][e][i] *= f;
       }
-      // P^T operands: hi = rnd(p), lo = rnd(p - hi) (p - hi exact in f32)
+      // P^T operands: term k = rnd(p - the terms before), each difference exact
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        if (AT == AT_BF16) {
-          ph[g][h] = pk_bf16(p[2 * h], p[2 * h + 1]);
-          pl[g][h] = pk_bf16(p[2 * h] - __uint_as_float(ph[g][h] << 16),
-                             p[2 * h + 1] - __uint_as_float(ph[g][h] & 0xffff0000u));
-        } else {
-          ph[g][h] = pk_f16(p[2 * h], p[2 * h + 1]);
-          pl[g][h] = pk_f16(p[2 * h] - h2f((f16_t)(ph[g][h] & 0xffffu)), p[2 * h + 1] - h2f((f16_t)(ph[g][h] >> 16)));
+        float r0 = p[2 * h], r1 = p[2 * h + 1];
+#pragma unroll
+        for (int k = 0; k < PT; k++) {
+          pt[g][k][h] = AT == AT_BF16 ? pk_bf16(r0, r1) : pk_f16(r0, r1);
+          r0 -= AT == AT_BF16 ? __uint_as_float(pt[g][k][h] << 16) : h2f((f16_t)(pt[g][k][h] & 0xffffu));
+          r1 -= AT == AT_BF16 ? __uint_as_float(pt[g][k][h] & 0xffff0000u) : h2f((f16_t)(pt[g][k][h] >> 16));
         }
       }
     }
@@ -128,8 +131,8 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
       const uint32_t a23 = __builtin_amdgcn_perm(w[3][e >> 1], w[2][e >> 1], sel);
 #pragma unroll
       for (int g = 0; g < GH; g++) {
-        acc[g][e] = mfma16x16<XT>(a01, a23, ph[g][0], ph[g][1], acc[g][e]);
-        acc[g][e] = mfma16x16<XT>(a01, a23, pl[g][0], pl[g][1], acc[g][e]);
+#pragma unroll
+        for (int k = 0; k < PT; k++) acc[g][e] = mfma16x16<XT>(a01, a23, pt[g][k][0], pt[g][k][1], acc[g][e]);
       }
     }
   };
