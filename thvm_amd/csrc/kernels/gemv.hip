@@ -21,16 +21,16 @@ typedef void (*gemv_fn)(ThvmGemvArgs);
 #define GEMV_PICKERS(X) \
   X(0, 0) X(0, 1) X(0, 2) X(1, 0) X(1, 1) X(1, 2) X(2, 0) X(2, 1) X(2, 2) X(3, 0) X(3, 1) X(3, 2) \
   X(2, 3) X(3, 3)
-#define GEMV_DECL(w, x) gemv_fn gemv_pick_##w##_##x(uint32_t M, int R, int U);
+#define GEMV_DECL(w, x) gemv_fn gemv_pick_##w##_##x(uint32_t M, int R, int U, uint32_t norm);
 GEMV_PICKERS(GEMV_DECL)
 #undef GEMV_DECL
 
 template <int WT>
-static gemv_fn pick_x(uint32_t xdt, uint32_t M, int R, int U, bool xsum = false) {
+static gemv_fn pick_x(uint32_t xdt, uint32_t M, int R, int U, uint32_t norm, bool xsum = false) {
   static_assert(WT_F32 == 0 && WT_FP8 == 3 && XD_BF16 == 0 && XD_F32 == 2 && XD_SUM4 == 3, "picker numbering");
   const int xd = xsum ? XD_SUM4
                : xdt == THVM_DT_BF16 ? XD_BF16 : xdt == THVM_DT_FP16 ? XD_F16 : xdt == THVM_DT_FP32 ? XD_F32 : -1;
-#define GEMV_CASE(w, x) if (WT == w && xd == x) return gemv_pick_##w##_##x(M, R, U);
+#define GEMV_CASE(w, x) if (WT == w && xd == x) return gemv_pick_##w##_##x(M, R, U, norm);
   GEMV_PICKERS(GEMV_CASE)
 #undef GEMV_CASE
   return nullptr;
@@ -230,10 +230,10 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   }
   gemv_fn f = nullptr;
   switch (a->wdt) {
-    case THVM_DT_FP32: f = pick_x<WT_F32>(a->xdt, Mk, R, U); break;
-    case THVM_DT_FP16: f = pick_x<WT_F16>(a->xdt, Mk, R, U); break;
-    case THVM_DT_BF16: f = pick_x<WT_BF16>(a->xdt, Mk, R, U, xsum); break;
-    case THVM_DT_FP8E4M3: f = pick_x<WT_FP8>(a->xdt, Mk, R, U, xsum); break;
+    case THVM_DT_FP32: f = pick_x<WT_F32>(a->xdt, Mk, R, U, a->norm); break;
+    case THVM_DT_FP16: f = pick_x<WT_F16>(a->xdt, Mk, R, U, a->norm); break;
+    case THVM_DT_BF16: f = pick_x<WT_BF16>(a->xdt, Mk, R, U, a->norm, xsum); break;
+    case THVM_DT_FP8E4M3: f = pick_x<WT_FP8>(a->xdt, Mk, R, U, a->norm, xsum); break;
   }
   if (!f) { snprintf(err, errlen, "gemv: no kernel instance (R=%d U=%d)", R, U); return -1; }
   uint32_t Gr = (a->N + R - 1) / R;

@@ -286,12 +286,15 @@ __device__ __forceinline__ void xs_put_f(unsigned char *xs, uint32_t K, uint32_t
 // the caller (bdim inside a loop was re-read from the implicit kernel
 // arguments with a vector load and a full wait, between the early x loads).
 // Returns false when wait() did.
-template <int WT, int XD, int M, int R, int U, bool COH, class WaitF, class XRowF, class HookF>
+// NK (standalone, M > 1): the fused norm at compile time (a.norm), else -1.
+template <int WT, int XD, int M, int R, int U, bool COH, int NK, class WaitF, class XRowF, class HookF>
 __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *xs_raw, float *red,
                                           const uint32_t g, const uint32_t gstride,
                                           const uint32_t nthr, const int nw, WaitF &&wait,
                                           XRowF &&xrow, HookF &&hook, const uint32_t bdim) {
   constexpr int E = WTr<WT>::E;
+  constexpr bool LN = NK == 2;
+  const uint32_t norm = NK < 0 ? a.norm : (uint32_t)NK;
   // LDS keeps x in its 16-bit storage type unless weights or x are f32
   constexpr int XT = (WT == WT_F32 || XD == XD_F32) ? XT_F32 : (XD == XD_BF16 || XD == XD_SUM4 ? XT_BF16 : XT_F16);
   static_assert(XD != XD_SUM4 || (M == 1 && !COH && WT != WT_F32), "summed x: one row, standalone");
@@ -310,9 +313,9 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   // are in flight (measured on gfx950 at M = 1: 1.2-1.3 us less per fused-norm
   // launch at the C4 shapes, f32 3072 x 768 with a LayerNorm 6.3 -> 5.4; no
   // change without a norm).  Not f32 x of two or three rows: with twice the
-  // registers per row they spill.  Row by row after the weights, as M > 1 had been, each
-  // row's loads waited for every load before them: at M = 3 the fused-norm
-  // gate/up (28672 x 4096 fp8) took 39.3 us against 30.6 now.  In the persistent
+  // registers per row they spill.  Row by row after the weights, as M > 1 had been,
+  // each row's loads waited for every load before them: at M = 3 the fused-norm
+  // gate/up (28672 x 4096 fp8) took 36.7 us against 27.1 now.  In the persistent
   // kernel (COH: x is written by other blocks of the launch and is read only
   // after wait()) the weights go first.
   // The weight loads of row group gg, chunk batch c0: raw buffer loads
@@ -389,14 +392,15 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   constexpr int XNM = M == 1 ? XN : 8;   // the same for several rows, standalone: of the rows taken as one list
   constexpr int NVN = XREG / VE;         // fused norm: x vectors per thread and row
   // rows normed per pass: all, but two at a time at M = 4 (four rows of x beside
-  // the gains and the weights in flight spilled)
-  constexpr int MP = M == 4 ? 2 : M;
+  // the gains and the weights in flight spilled) and one at a time of three f32
+  // rows behind a LayerNorm (beside its gains and biases they spilled)
+  constexpr int MP = M == 4 ? 2 : LN && M == 3 && XD == XD_F32 ? 1 : M;
   constexpr int NPRE = XNM > MP * NVN ? XNM : MP * NVN;
   // x as raw 16-byte vectors, requested before the weights: with a norm, row
   // m's vectors tid + j*nthr at [m*NVN + j]; without, the first pass over the
   // rows' list, vectors threadIdx.x + j*bdim (clamped indices; vectors past
   // the rows are never stored)
-  constexpr bool XPRE = !COH && (XD != XD_F32 || M == 1 || M == 4) && XD != XD_SUM4;
+  constexpr bool XPRE = !COH && (XD != XD_F32 || M == 1 || M == 4 || LN) && XD != XD_SUM4;
   const uint32_t NVM = (uint32_t)M * NVt;
   // vector f of the rows' list -> its row and its vector there
   auto row_of = [&](uint32_t f, uint32_t &v) {
@@ -426,7 +430,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   if (XPRE) {
     // (uniform skips of vectors past the rows for every thread: a K below the
     // staging's reach needs fewer loads)
-    if (a.norm == 0) {
+    if (norm == 0) {
 #pragma unroll
       for (int j = 0; j < XNM; j++) {
         if (j * bdim >= NVM) break;
@@ -451,8 +455,8 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   // own (clamped indices; lanes past the row never use them)
   float gw[NVN][VE], gb[NVN][VE];
   auto load_gains = [&] {
-    if (XSUM || a.norm == 0) return;
-    const bool hw = a.norm_w != nullptr, hb = a.norm == 2 && a.norm_b != nullptr;
+    if (XSUM || norm == 0) return;
+    const bool hw = a.norm_w != nullptr, hb = norm == 2 && a.norm_b != nullptr;
 #pragma unroll
     for (int j = 0; j < NVN; j++) {
       const uint32_t v = tid + j * nthr, vc = v < NVt ? v : 0;
@@ -460,7 +464,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       for (int i = 0; i < VE; i += 4) {
         const float4 t = hw ? *(const float4 *)(a.norm_w + vc * VE + i) : make_float4(1.f, 1.f, 1.f, 1.f);
         gw[j][i] = t.x; gw[j][i + 1] = t.y; gw[j][i + 2] = t.z; gw[j][i + 3] = t.w;
-        if (M == 1 || COH) {
+        if (M == 1 || COH || LN) {
           const float4 u = hb ? *(const float4 *)(a.norm_b + vc * VE + i) : make_float4(0.f, 0.f, 0.f, 0.f);
           gb[j][i] = u.x; gb[j][i + 1] = u.y; gb[j][i + 2] = u.z; gb[j][i + 3] = u.w;
         }
@@ -475,8 +479,12 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   // 2 x staged, 3 first weight batch consumed, 4 wave 0's rows done
   uint64_t *const clk = COH ? nullptr : a.clk;
   pclk(clk, a.clk_cap, 0);
+  // a LayerNorm over several rows goes before the weights altogether: its gains
+  // and biases do not fit beside them in 128 registers, and biases loaded after
+  // the weights wait for all of them, a round trip per row and vector (4096 x
+  // 4096 fp16, M = 2 and 4: 15.3 and 24.5 us so, 9.8 and 14.7 now)
   const bool early = !COH || (threadIdx.x >> 6) != 0;
-  if (early) load_batch(g, 0);
+  if (early && !LN) load_batch(g, 0);
   if (!wait()) return false;
   if (!early) load_batch(g, 0);
   if (!XPRE) load_gains();
@@ -505,7 +513,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       *(uint32_t *)(xs_raw + (size_t)hi * 2u) = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
     }
   } else if constexpr (!COH && M > 1) {
-    if (a.norm == 0) {
+    if (norm == 0) {
       // no reduction: every thread of the block stages, XNM vectors of x in
       // flight per thread before the first LDS store
       for (uint32_t f0 = threadIdx.x; f0 < NVM; f0 += XNM * bdim) {
@@ -552,7 +560,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       float mean[MP], s2[MP];
 #pragma unroll
       for (int m = 0; m < MP; m++) mean[m] = s2[m] = 0.0f;
-      if (a.norm == 2) {
+      if (LN) {
 #pragma unroll
         for (int m = 0; m < MP; m++)
 #pragma unroll
@@ -561,7 +569,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
             xdec<XD>(xpre[m * NVN + j], xf);
 #pragma unroll
             for (int i = 0; i < VE; i++) mean[m] += xf[i];
-            }
+          }
         block_sum_m<MP>(mean, red, nw);
 #pragma unroll
         for (int m = 0; m < MP; m++) mean[m] = mean[m] * invK;
@@ -596,7 +604,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
               // (x - mean) * inv * w (+ b), the norm kernel's own formula
               val[i] = (val[i] - mean[m]) * inv;
               if (a.norm_w) val[i] = val[i] * gw[j][i];
-              if (a.norm == 2 && a.norm_b) val[i] = val[i] + a.norm_b[v * VE + i];
+              if (LN && a.norm_b) val[i] = val[i] + gb[j][i];
             }
             xs_put_f<XD, XT, E>(xs_raw, K, C, mb + m, v, val);
           }
@@ -607,7 +615,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
   for (int m = 0; m < M; m++) {
     const void *xr = xrow(m);
     constexpr bool pre = XPRE;           // (M = 1) the row is already in xpre
-    if (a.norm == 0) {
+    if (norm == 0) {
       // no reduction: every thread of the block stages, XN vectors of x in
       // flight per thread before the first LDS store
       for (uint32_t v0 = threadIdx.x; v0 < NVt; v0 += XN * bdim) {
@@ -640,7 +648,7 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
       }
       const float invK = 1.0f / (float)K;
       float mean = 0.0f, s1 = 0.0f, s2 = 0.0f;
-      if (a.norm == 2) {
+      if (norm == 2) {
 #pragma unroll
         for (int j = 0; j < NV; j++)
 #pragma unroll
@@ -667,12 +675,16 @@ __device__ __forceinline__ bool gemv_core(const ThvmGemvArgs &a, unsigned char *
             // (x - mean) * inv * w (+ b), the norm kernel's own formula
             val[i] = (xv[j][i] - mean) * inv;
             if (a.norm_w) val[i] = val[i] * gw[j][i];
-            if (a.norm == 2 && a.norm_b) val[i] = val[i] + gb[j][i];
+            if (norm == 2 && a.norm_b) val[i] = val[i] + gb[j][i];
           }
           xs_put_f<XD, XT, E>(xs_raw, K, C, m, v, val);
         }
       }
     }
+  }
+  if (LN) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_batch(g, 0);
   }
   if (PRE && M > 1) load_pre();
   __syncthreads();
