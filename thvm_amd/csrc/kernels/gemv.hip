@@ -187,28 +187,35 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
     }
   }
   // two rows per wave where a row fills at most half a batch of chunks (half
-  // the lanes would idle) and one row per wave would take more than one block
-  // per CU, each staging x: measured on gfx950, 102400 x 2048 fp8 (the C5 LM
-  // head) 53.5 -> 38.9 us, 3648 x 2048 with a fused norm 5.9 -> 5.5 us at M = 1
-  // and 9.9 -> 9.1 at 4; 2048 x 2048 (256 blocks) 3.9 us stays.  A row's lanes
-  // and chunk order are unchanged, so the sums are bit-identical.
-  if (!a->tune_r && R == 1 && a->N % 2 == 0 && a->N > 2048 && a->M <= 4 && (uint64_t)a->K * wsz / 16 <= 128) {
+  // the lanes would idle) and that either still makes at most 256 blocks behind a
+  // norm each of them computes, or leaves many.  Two rows over one, M = 1..4, fp8
+  // and fp16 rows of 768..2048 bytes: with a norm 0.80..0.98 of the time at N =
+  // 2304..4096, 1.05..1.28 at 4608..6144 (a second round of blocks, half full),
+  // 0.95..1.10 up to 14336, 0.79..0.94 from 16384; without one 1.02..1.25 up to
+  // 4096, 0.82..1.00 from 16384.  A row's lanes and chunk order are unchanged, so
+  // the sums are bit-identical.
+  if (!a->tune_r && R == 1 && a->N % 2 == 0 && a->M <= 4 && (uint64_t)a->K * wsz / 16 <= 128 &&
+      (a->N >= 16384 || (a->norm && a->N > 2048 && a->N <= 4096))) {
     R = 2;
   }
-  // two rows per wave too where one per wave takes more than 256 blocks of 8
-  // waves and two fit in 256, over rows of less than a full batch of chunks: one
-  // block per CU (3072 x 768 f32 with a LayerNorm: 6.96 -> 6.25 us with the wave
-  // count below; full-batch rows, 4096 x 4096 fp8, are faster at 16 waves)
+  // behind a LayerNorm of one row also over rows of less than a full batch of
+  // chunks, as with the wave count below two rows per wave are one block per CU
+  // (3072 x 768 f32: 6.96 -> 6.25 us; without a norm 3072 x 1600 fp16 4.4 -> 4.8)
   if (!a->tune_r && R == 1 && a->M == 1 && a->N % 2 == 0 && a->N > 2048 && a->N <= 4096 &&
-      (uint64_t)a->K * wsz / 16 < 256 && a->norm != 1) {
+      (uint64_t)a->K * wsz / 16 < 256 && a->norm == 2) {
     R = 2;
   }
-  // three or four x rows over long weight rows (>= 768 chunks): two rows per
-  // wave share each x read from LDS (measured on gfx950 at the C4 down shape,
-  // 14336-wide fp8 rows: M = 3 21.2 -> 17.1 us, M = 4 23.3 -> 18.8; at M = 2 one
-  // row is faster, 14.0 against 15.8, and so it is with f32 operands, 768 x 3072
-  // at M = 3 7.2 against 10.6); bit-identical sums
-  if (!a->tune_r && R == 1 && Mk >= 3 && a->xdt != THVM_DT_FP32 && a->wdt != THVM_DT_FP32 && a->N % 2 == 0 && (uint64_t)a->K * wsz / 16 >= 768) R = 2;
+  // three or four 16-bit x rows over weight rows of 768 to 1023 chunks: two rows
+  // per wave share each x read from LDS where that fills one round of blocks or
+  // leaves many (14336-wide fp8 rows, M = 3 and 4, two rows over one: N = 3072
+  // 0.90 and 0.87 of the time, 4096 0.95 and 0.92, from 8192 on 0.78..0.88; but
+  // 1.05 at 5120 and 6144, 1.27..1.37 up to 2048, and 1.07..1.40 at most N over
+  // rows of 1024 chunks and more); bit-identical sums
+  if (!a->tune_r && R == 1 && Mk >= 3 && a->xdt != THVM_DT_FP32 && a->wdt != THVM_DT_FP32 && a->N % 2 == 0 &&
+      ((a->N > 2048 && a->N <= 4096) || a->N >= 8192) && (uint64_t)a->K * wsz / 16 >= 768 &&
+      (uint64_t)a->K * wsz / 16 < 1024) {
+    R = 2;
+  }
   if (a->tune_r) {
     if (a->tune_r != 1 && a->tune_r != 2) { snprintf(err, errlen, "gemv: r must be 1 or 2"); return -1; }
     if ((pairs && a->tune_r == 1) || a->N % a->tune_r) { snprintf(err, errlen, "gemv: r=%u does not tile N/epilogue", a->tune_r); return -1; }
@@ -256,11 +263,14 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   // fewer than 8 waves where that still is one block per CU or less: the rows
   // spread over every CU (768 x 3072 f32, 96 blocks of 8 waves: 6.02 -> 5.65 us
   // at 3; 2304 x 768 with a LayerNorm in pairs, 144 blocks: 6.52 -> 5.64 at 6).
+  // Three waves only where they stage x in one pass, four above (256..768 rows
+  // of 8192..28672 fp8: 4 waves 0.92..1.01 of the time of 8, 3 waves 0.96..1.03).
   // Not with a fused RMSNorm, whose sum is in the order of a 512-thread block
   // (the persistent step's).
   if (!a->tune_waves && Mk == 1 && chunks == 1 && !xsum && a->norm != 1 && Gr <= 2048) {
     const uint32_t w = (Gr + 255) / 256, wmin = a->norm ? (uint32_t)((a->K + XREG * 64 - 1) / (XREG * 64)) : 1u;
-    const uint32_t lo = wmin > 3 ? wmin : 3;
+    const uint32_t pass3 = 4u * 64u * 3u * (a->xdt == THVM_DT_FP32 ? 4u : 8u);
+    const uint32_t few = a->K <= pass3 ? 3 : 4, lo = wmin > few ? wmin : few;
     waves = w < lo ? lo : w > 8 ? 8 : w;
   }
   if (Mk > 1 && waves > 8) waves = 8;   // the instances' block limit; the sums do not depend on it
