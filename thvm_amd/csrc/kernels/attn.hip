@@ -609,23 +609,25 @@ static bool attn_mf_can(const ThvmAttnArgs *a) {
 // One launch in which a block takes every chunk of its (row, kv head) and
 // writes the output itself, as fused = 2 picks it: no partials, and none of
 // the ~3 us that their hand-off (or a second launch) takes.  What it gives up
-// is the chunks running side by side, so the line lies at a block's work,
-// n_split G hd products a cache row; from half the CUs up in blocks the other
-// forms have nothing left to spread over, and it wins up to 16 chunks.
-// Measured on gfx950, us per launch in a graph, the form picked before -> this
-// (a full cache; at half the length it gains more):
-//   fp16 hd 64 G 1, 8 rows x 25 heads: 3 chunks 8.6 -> 5.1, 8 chunks 11.1 ->
-//   7.7, 16 chunks 16.1 -> 11.5; 12 heads: 8 chunks 7.1 -> 5.3, 9 chunks 7.1
-//   -> 6.2, but 16 chunks 7.8 -> 9.4; f32, 12 heads: 9 chunks 7.7 -> 8.0;
-//   bf16 hd 128 G 4: 3 chunks x 32 9.5 -> 9.1, 8 chunks x 256 23.1 -> 17.5,
-//   but 8 chunks x 64 12.3 -> 16.2; hd 128 G 2: 8 chunks x 32 9.4 -> 10.8.
+// is the chunks running side by side, so it is for calls whose (row, kv head)
+// pairs fill the chip by themselves.  Measured on gfx950, this form's time over
+// that of the form picked else, in a graph, a full cache / half of one:
+//   2 to 8 chunks, G 1, 2, 4, hd 64 (fp16, f32) and 128 (bf16):
+//     8..64 pairs   1.05..1.97 / 0.93..1.31 (bf16 hd 128 G 1 has faster spots)
+//     96, 128       0.92..1.30 / 0.70..1.07
+//     192..256      0.78..0.99 / 0.62..0.87
+//   9 to 16 chunks, G 1:
+//     8..64 pairs   fp16 hd 64 9 chunks 0.81..0.92 / 0.64..0.71, 12 chunks
+//                   0.96..1.10 / 0.71..0.79, 16 1.10..1.33; others 0.85..1.86
+//     96..256       0.66..1.01 / 0.55..0.89
+//   G 4 (9 to 16 chunks, 16 bits): 1.00..3.47 / 0.91..2.19.
 // The forced one-launch form (fused = 1) keeps the split of auto_cpb.
 static bool attn_whole(const ThvmAttnArgs *a) {
   const uint32_t G = a->Hkv ? a->H / a->Hkv : 0, bh = a->B * a->Hkv;
   if (a->fused != 2 || a->mf == 1 || (a->cpb && a->cpb < a->n_split) || (G != 1 && G != 2 && G != 4)) return false;
-  const uint64_t work = (uint64_t)a->n_split * G * a->hd;
-  if (a->n_split <= 8) return work <= 1536 || bh >= 128;
-  return G == 1 && a->n_split <= 16 && (bh >= 128 || (a->cdt != THVM_DT_FP32 && work <= 768));
+  if (a->n_split <= 8) return bh >= 192;
+  return G == 1 && a->n_split <= 16 &&
+         (bh >= 96 || (a->cdt != THVM_DT_FP32 && a->hd == 64 && a->n_split <= 10));
 }
 
 // split and merge in one launch: asked for, or the shape's pick
