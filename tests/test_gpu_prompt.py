@@ -291,3 +291,32 @@ def test_attn_prompt_keeps_p_in_f32(hip, H, Hkv, hd):
         want = (p / p.sum(-1, keepdims=True)) @ vf[h * Hkv // H]
         off += (O.encode(want.astype(np.float32), dt) != got[:, h]).sum()
     assert off <= 5e-4 * got.size, off / got.size
+
+
+@pytest.mark.parametrize("dt,bits", [(DT_BF16, 0x7F80), (DT_BF16, 0xFFC0), (DT_F16, 0x7C00), (DT_F16, 0xFC00), (DT_F16, 0x7E01)])
+@pytest.mark.parametrize("H,Hkv,hd", [(4, 2, 64), (3, 3, 128)])
+@pytest.mark.parametrize("T,pos,at", [(40, 0, 7), (33, 21, 15), (48, 16, 47), (5, 14, 0)])
+def test_attn_prompt_later_v_not_finite(hip, dt, bits, H, Hkv, hd, T, pos, at):
+    """An infinity or NaN in one value of a chunk row's V reaches that row's
+    position and the ones after it, in that value alone; the positions before
+    it, which share its tile of rows, keep their bits."""
+    say(f"case: attn_prompt V not finite dt={dt} bits={bits:x} H={H} hd={hd} T={T} pos={pos} at={at}")
+    rng = np.random.default_rng(T + pos + at)
+    ms, scale, d, kvh = pos + T + 3, float(np.float32(1 / np.sqrt(hd))), hd - 3, Hkv - 1
+    q, k, v = (O.encode(rng.standard_normal(s).astype(np.float32), dt) for s in ((1, T, H, hd), (1, Hkv, ms, hd), (1, Hkv, ms, hd)))
+    outs = []
+    for x in (None, bits):
+        vv = v.copy()
+        if x is not None:
+            vv[0, kvh, pos + at, d] = x
+        out = hip.Buffer(T * H * hd * 2)
+        hip.builtin("attn_prompt", [out, up(hip, q), up(hip, k), up(hip, vv), up(hip, np.array([pos + 1], np.int32))],
+                    b=1, t=T, h=H, hkv=Hkv, hd=hd, maxseq=ms, dt=dt, scale=scale)
+        outs.append(out.read(np.uint16).reshape(T, Hkv, H // Hkv, hd))
+    hit = np.zeros(outs[0].shape, bool)
+    hit[at:, kvh, :, d] = True
+    assert np.array_equal(outs[0][~hit], outs[1][~hit])
+    f = O.decode(outs[1][hit], dt)
+    assert not np.isfinite(f).any()
+    if bits in (0x7F80, 0x7C00, 0xFC00) and at // 16 == (T - 1) // 16:
+        assert np.all(np.isinf(f) & (np.signbit(f) == (bits > 0x7FFF)))

@@ -35,6 +35,7 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
   constexpr int XT = AT == AT_BF16 ? GX_BF16 : GX_F16;
   constexpr int KS = HD / 32, NC = HD / 8, PT = AT == AT_BF16 ? 3 : 2;   // PT: 16-bit terms of p
   constexpr float PS = AT == AT_BF16 ? 1.0f : 16384.0f;
+  constexpr uint32_t EXP = AT == AT_BF16 ? 0x7f80u : 0x7c00u;              // all ones: infinite or NaN
   extern __shared__ __align__(16) float apl[];
   float(*const wacc)[GH * 16][HD + 4] = (float(*)[GH * 16][HD + 4])apl;      // [wave][head, position][d]
   __shared__ float wm[AP_WAVES][GH * 16], wl[AP_WAVES][GH * 16];
@@ -80,9 +81,12 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[g][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
+  int tbad = -1;                                          // see tile: a masked tile with V that is not finite
+  float pbad[GH][4] = {};
   auto tile = [&](int buf, int t) {
     const int32_t rb = 16 * t + 4 * lg;
     uint32_t pt[GH][PT][2];
+    float p[GH][4];
 #pragma unroll
     for (int g = 0; g < GH; g++) {
       f32x4_t sc = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -96,10 +100,9 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
       mx = fmaxf(mx, xor32_f(mx));
       const float mn = fmaxf(m[g], mx);
       const float f = m[g] == -INFINITY ? 0.0f : fexp2(m[g] - mn);
-      float p[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) p[i] = sv[i] == -INFINITY ? 0.0f : fexp2(sv[i] - mn) * PS;
-      l[g] = l[g] * f + ((p[0] + p[1]) + (p[2] + p[3]));
+      for (int i = 0; i < 4; i++) p[g][i] = sv[i] == -INFINITY ? 0.0f : fexp2(sv[i] - mn) * PS;
+      l[g] = l[g] * f + ((p[g][0] + p[g][1]) + (p[g][2] + p[g][3]));
       m[g] = mn;
       if (__builtin_amdgcn_ballot_w64(f != 1.0f)) {
 #pragma unroll
@@ -110,19 +113,42 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
       // P^T operands: term k = rnd(p - the terms before), each difference exact
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        float r0 = p[2 * h], r1 = p[2 * h + 1];
+        float x0 = p[g][2 * h], x1 = p[g][2 * h + 1];
 #pragma unroll
         for (int k = 0; k < PT; k++) {
-          pt[g][k][h] = AT == AT_BF16 ? pk_bf16(r0, r1) : pk_f16(r0, r1);
-          r0 -= AT == AT_BF16 ? __uint_as_float(pt[g][k][h] << 16) : h2f((f16_t)(pt[g][k][h] & 0xffffu));
-          r1 -= AT == AT_BF16 ? __uint_as_float(pt[g][k][h] & 0xffff0000u) : h2f((f16_t)(pt[g][k][h] >> 16));
+          pt[g][k][h] = AT == AT_BF16 ? pk_bf16(x0, x1) : pk_f16(x0, x1);
+          x0 -= AT == AT_BF16 ? __uint_as_float(pt[g][k][h] << 16) : h2f((f16_t)(pt[g][k][h] & 0xffffu));
+          x1 -= AT == AT_BF16 ? __uint_as_float(pt[g][k][h] & 0xffff0000u) : h2f((f16_t)(pt[g][k][h] >> 16));
         }
       }
     }
-    const uint32_t w[4][4] = {{vb[buf][0].x, vb[buf][0].y, vb[buf][0].z, vb[buf][0].w},
-                              {vb[buf][1].x, vb[buf][1].y, vb[buf][1].z, vb[buf][1].w},
-                              {vb[buf][2].x, vb[buf][2].y, vb[buf][2].z, vb[buf][2].w},
-                              {vb[buf][3].x, vb[buf][3].y, vb[buf][3].z, vb[buf][3].w}};
+    uint32_t w[4][4] = {{vb[buf][0].x, vb[buf][0].y, vb[buf][0].z, vb[buf][0].w},
+                        {vb[buf][1].x, vb[buf][1].y, vb[buf][1].z, vb[buf][1].w},
+                        {vb[buf][2].x, vb[buf][2].y, vb[buf][2].z, vb[buf][2].w},
+                        {vb[buf][3].x, vb[buf][3].y, vb[buf][3].z, vb[buf][3].w}};
+    // A masked score is a zero p, but zero times a V that is not finite (an
+    // overflow in a later position) is NaN: in the tiles that some column of the
+    // block masks such values leave the products, and after the last tile the
+    // columns that do see their rows add them one by one.  Those tiles are the
+    // block's last two at most, so a wave's is its last: its p are the final ones.
+    if (16 * t + 15 > pos + (int32_t)t0) {                // wave-uniform
+      uint32_t bad = 0;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const uint32_t lo = (w[j][k] & EXP) == EXP ? 0xffffu : 0u, hi = (w[j][k] >> 16 & EXP) == EXP ? 0xffff0000u : 0u;
+          bad |= lo | hi;
+          w[j][k] &= ~(lo | hi);
+        }
+      if (__builtin_amdgcn_ballot_w64(bad != 0)) {
+        tbad = t;                                         // (the wave's last tile)
+#pragma unroll
+        for (int g = 0; g < GH; g++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) pbad[g][i] = p[g][i];
+      }
+    }
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       // column 8 lc + e of rows 0..3: the low (e even) or high half of dword e/2
@@ -151,6 +177,31 @@ __global__ __launch_bounds__(AP_THREADS, 2) void k_attn_prompt(ThvmAttnArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     issue(1, t + 3 * AP_WAVES);
     __builtin_amdgcn_sched_barrier(0);
+  }
+  if (tbad >= 0) {                                        // wave-uniform
+#pragma unroll 1
+    for (int jj = 0; jj < 4; jj++)                        // rows 16 tbad + 4 jj + i: their p are in lane group jj
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int32_t r = 16 * tbad + 4 * jj + i;
+        float pr[GH];
+#pragma unroll
+        for (int g = 0; g < GH; g++) pr[g] = __shfl(pbad[g][i], lc + 16 * jj);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {                     // this lane's d = 8 (4 lg + q) + e
+          const int mm = 4 * lg + q;
+          const uint4 v = buf_ld16(vrs, r < r1 && r < lim && mm < NC ? (uint32_t)(r * HD + 8 * mm) * 2 : BUF_OOB);
+          const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const uint32_t h = e & 1 ? vw[e >> 1] >> 16 : vw[e >> 1] & 0xffffu;
+            if ((h & EXP) != EXP) continue;
+            const float x = AT == AT_BF16 ? __uint_as_float(h << 16) : h2f((f16_t)h);
+#pragma unroll
+            for (int g = 0; g < GH; g++) acc[g][e][q] += pr[g] * x;
+          }
+        }
+      }
   }
 #pragma unroll
   for (int g = 0; g < GH; g++) {
