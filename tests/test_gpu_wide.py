@@ -261,3 +261,29 @@ def test_wide_gemm_empty_and_huge_shapes_refused(hip):
     for m, n, k in ((65, 0, 64), (0, 64, 64), (65, 64, 0), (2 ** 32 - 1, 64, 64), (65, 2 ** 32 - 1, 64), (2 ** 32 - 1, 2 ** 32 - 1, 64)):
         with pytest.raises(hip.ThvmHipError):
             hip.builtin("gemv", [b, b, b, b], m=m, n=n, k=k, wt=DT_BF16, xt=DT_BF16, yt=DT_BF16, ws=1)
+
+
+@pytest.mark.parametrize("wx", [(DT_FP8, DT_BF16), (DT_BF16, DT_BF16), (DT_F16, DT_F16)])
+@pytest.mark.parametrize("K", [1024, 1600, 4096, 14336])
+def test_wide_gemm_sums_as_exact_as_k_gemm(hip, wx, K):
+    """The f32 sums' error against float64 (2-norm over the result's) is no
+    larger than that of k_gemm, whose place the wide GEMM takes above 16 rows
+    and whose waves each sum an eighth of K: at every tile, K unsplit, where a
+    wave's slice is longest, and split."""
+    (wdt, xdt), M, N = wx, 60, 256
+    say(f"case: wide gemm sums wdt={wdt} K={K}")
+    x, w, scale, xf, wf = case(np.random.default_rng(N + K), wdt, xdt, M, N, K)
+    ref = xf @ wf.T
+    args, ws = [up(hip, x), up(hip, w), *([up(hip, scale)] if scale is not None else [])], hip.Buffer(WS)
+
+    def err(extra, **kw):
+        y = hip.Buffer(M * N * 4)
+        hip.builtin("gemv", [y, *args, *extra], m=M, n=N, k=K, wt=wdt, xt=xdt, yt=DT_F32, **kw)
+        return np.linalg.norm(y.read(np.float32).reshape(M, N) - ref) / np.linalg.norm(ref)
+
+    # (seq, which the plain store does not read, takes the wide GEMM at any shape)
+    bar = err([])
+    for r in (1, 2, 4):
+        for blocks in (1, 2):
+            e = err([ws], ws=1, seq=1, r=r, blocks=blocks)
+            assert e <= bar, (r, blocks, e, bar)

@@ -14,17 +14,22 @@ WIDE_PICKERS(WIDE_DECL)
 // Where this kernel takes over from k_gemm (16 < M <= 64; above it is the only
 // one).  k_gemm's x reads grow with M K N / (16 NT), this one pays a longer
 // chain per block (a barrier per 128 k, the split hand-off).  Measured on
-// gfx950, cold fp8 weights in a graph, k_gemm against this kernel, us:
-//   28672 x 4096  M 17 33.4 / 23.8   M 60 50.0 / 31.5      wide N
-//   14336 x 2048  M 17 10.6 /  8.0   M 60 16.3 / 11.2
-//   32000 x 1024  M 17 13.7 /  9.2   M 60 20.1 / 11.7
-//    4096 x 14336 M 17 17.8 / 14.5   M 60 33.6 / 19.2      long K
-//    2048 x 8192  M 17 10.4 /  9.1   M 60 18.4 / 12.2
-//    6144 x 4096  M 17 11.5 / 11.5   M 60 18.7 / 16.4      middling: by M
-//    4096 x 4096  M 17  7.5 /  8.2   M 60 11.9 / 10.5
-//    2048 x 4096  M 17  7.2 /  7.2   M 60 11.4 /  9.6
-//    6400 x 1600  M 17  6.4 /  7.0   M 60  9.3 /  9.5      small: k_gemm
-//    1600 x 1600  M 17  5.1 /  6.5   M 60  7.1 /  8.8
+// gfx950, cold tiled fp8 weights in a graph, k_gemm / this kernel, us:
+//                  M 8          M 16         M 17         M 60
+//   28672 x 4096   22.0 / 21.2  23.0 / 21.3  28.5 / 21.4  40.5 / 26.1   wide N
+//   14336 x 2048    9.3 /  7.5   9.8 /  7.8  10.1 /  7.8  16.1 / 11.1
+//   32000 x 1024   10.9 /  8.7  11.9 /  8.9  13.3 /  8.9  20.0 / 11.7
+//    4096 x 14336  13.6 / 13.6  15.5 / 13.9  17.1 / 13.9  33.1 / 18.7   long K
+//    1600 x 6400    7.6 /  8.4   8.4 /  8.5   9.4 /  8.5  16.3 / 11.2
+//    2048 x 8192    8.0 /  9.2   9.0 /  9.3  10.2 /  9.3  18.4 / 11.8
+//    6144 x 4096    7.6 /  8.4   8.1 /  8.8   9.2 /  8.8  14.1 / 12.4   middling: by M
+//    4096 x 4096    6.2 /  8.0   6.6 /  8.1   7.4 /  8.1  11.8 / 10.4
+//    2048 x 4096    5.6 /  7.2   6.0 /  7.3   7.0 /  7.3  11.4 /  9.6
+//    6400 x 1600    5.3 /  6.8   5.6 /  6.9   6.3 /  6.9   9.2 /  9.4   small: k_gemm
+//    1600 x 1600    4.2 /  6.3   4.3 /  6.5   5.0 /  6.5   7.1 /  8.9
+// At 16 rows and fewer the widest N gain 4..25% too, and a long K 10% at 16;
+// the line stays at 16 because k_gemm also takes a norm ahead of the product
+// there, and a decoder of 5 to 16 rows holds no workspace.
 extern "C" int thvm_k_gemm_wide_use(const ThvmGemvArgs *a) {
   if (a->seq) return 1;
   if (a->M <= 16) return 0;

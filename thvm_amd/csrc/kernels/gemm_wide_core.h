@@ -8,16 +8,28 @@
 // What bounds it: k_gemm (gemm.hip) gives each wave of a block its own K slice
 // and so its own x, and every block reads all of x for the 16..64 weight rows
 // it owns: at 64 rows the x reads from L2 are 8 times the weight bytes of the
-// 14336-wide down projection (470 MB against 59).  Here the 4 waves of a block
-// own different weight rows and share one x tile in LDS, and K is split over
-// blocks where the weight rows alone would not fill the chip, so a block reads
-// only its K slice of x for 64 NT weight rows.
-//   * tile: BM = 16 MT x rows by BN = 64 NT weight rows, wave w the 16-row
-//     groups w NT .. w NT + NT - 1 of the block; per 64-k step a wave reads 2 MT
-//     x operands from LDS for 2 NT MT MFMAs;
-//   * x chunks of 128 k, two LDS buffers: the next chunk is stored while this
-//     one is consumed (one barrier per chunk) and the one after is in flight in
-//     registers; weights 4 steps (16 NT bytes x WB per lane each) ahead;
+// 14336-wide down projection (470 MB against 59).  Here the 8 waves of a block
+// share one x tile in LDS, 4 along the weight rows by 2 along k, and K is split
+// over blocks where the weight rows alone would not fill the chip, so a block
+// reads only its K slice of x for 64 NT weight rows.
+//   * tile: BM = 16 MT x rows by BN = 64 NT weight rows, waves w and w + 4 the
+//     16-row groups w NT .. w NT + NT - 1 of the block, one on the even and one
+//     on the odd 64-k steps; per step a wave reads 2 MT x operands from LDS for
+//     2 NT MT MFMAs, and at the end the two halves of k meet through LDS;
+//   * x chunks of 128 k (a step for each wave of a pair), two LDS buffers: the
+//     next chunk is stored while this one is consumed (one barrier per chunk);
+//     x and weights are both requested U = 4 chunks ahead (2 where the widest
+//     tile's registers leave no more: x 8 MT, weights 4 NT x WB of them a chunk);
+//   * sums in two levels: an MFMA chain runs over 4 chunks (16-bit weights: 1) and
+//     is then added to the tile's sums.  Error against float64 of the f32 sums
+//     (2-norm over the result's, 1e-7; K = 1024 .. 14336, K unsplit, the worst):
+//                          fp8 W          bf16 W         fp16 W
+//       one chain          0.74 .. 2.99   1.28 .. 5.31   1.48 .. 5.42
+//       two levels         0.64 .. 1.16   0.76 .. 2.00   0.85 .. 2.03
+//       k_gemm (8 slices)  0.68 .. 1.40   0.83 .. 2.59   0.95 .. 2.76
+//       the GEMV           0.59 .. 0.83   0.67 .. 1.16   0.86 .. 2.03
+//     It costs up to 4% (28672 x 4096 fp8, M = 512, tiled: 141 -> 147 us; M = 60
+//     26.0 -> 26.1);
 //   * rows padded by 16 bytes: the 16 rows of one operand read fall in
 //     different banks;
 //   * splits > 1: each block stores its f32 tile with system-scope stores and
@@ -192,7 +204,10 @@ __global__ __launch_bounds__(GW_THREADS, 2) void k_gemm_wide(ThvmGemvArgs a) {
   __shared__ float ssum[NM ? 16 * MT : 1];
   __shared__ uint32_t last;
   static_assert(!NM || XT == GX_BF16, "the fused norm stages bf16 x");
-  constexpr int BM = 16 * MT, WB = WT == GW_FP8 ? 1 : 2, U = 4;
+  // U chunks in flight (two where the tile's registers leave no more), F chunks a
+  // chain, T chunks a turn of the loop
+  constexpr int BM = 16 * MT, WB = WT == GW_FP8 ? 1 : 2, U = NT == 4 && MT == 4 ? 2 : 4;
+  constexpr int F = WT == GW_FP8 ? 4 : 1, T = 4;
   constexpr int NI = BM * 16 / GW_THREADS;                 // 16-byte x pieces per thread and chunk
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane((tid >> 6) % GW_NWAVES), kg = __builtin_amdgcn_readfirstlane(tid >> 6) / GW_NWAVES;
@@ -224,7 +239,13 @@ __global__ __launch_bounds__(GW_THREADS, 2) void k_gemm_wide(ThvmGemvArgs a) {
                              (uint32_t)(((uint64_t)(xrows - 1) * a.ldx + K) * 2));
   const buf_t grs = buf_rsrc(NM ? (const void *)a.norm_w : (const void *)a.x, NM ? K * 4u : 0u);
 
-  f32x4_t acc[NT][MT];
+  // chained through the accumulator alone, a row's sum takes a rounding per 32 k
+  // of its slice; so a chain starts anew every F chunks and is added to the sums
+  // of the ones before.  F is where the error is least of what the registers
+  // allow: 16-bit weights, whose products round more in a chain, fold every chunk,
+  // which needs no second set of accumulators either (with it the widest tile
+  // spilled: 4096 x 14336 bf16, M = 512, 172 -> 207 us)
+  f32x4_t acc[NT][MT], ch[NT][MT];
 #pragma unroll
   for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -278,7 +299,7 @@ __global__ __launch_bounds__(GW_THREADS, 2) void k_gemm_wide(ThvmGemvArgs a) {
     for (int i = 0; i < NI; i++)
       *(uint4 *)(xs + (size_t)buf * (BM * GW_XROW) + (xr + XRP * i) * GW_XROW + xk * 2) = xv.x[i];
   };
-  auto compute = [&](int buf, int so, int u) {
+  auto compute = [&](int buf, int so, int u, bool first) {
     const unsigned char *xb = xs + (size_t)buf * (BM * GW_XROW) + li * GW_XROW + so * 128 + lg * 32;
     uint4 B[MT][2];
 #pragma unroll
@@ -300,8 +321,13 @@ __global__ __launch_bounds__(GW_THREADS, 2) void k_gemm_wide(ThvmGemvArgs a) {
       }
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
-        acc[t][mt] = mfma16<XT>(A0, B[mt][0], acc[t][mt]);
-        acc[t][mt] = mfma16<XT>(A1, B[mt][1], acc[t][mt]);
+        if constexpr (F == 1) {
+          const f32x4_t c = mfma16<XT>(A0, B[mt][0], f32x4_t{0.f, 0.f, 0.f, 0.f});
+          acc[t][mt] += mfma16<XT>(A1, B[mt][1], c);
+        } else {
+          ch[t][mt] = mfma16<XT>(A0, B[mt][0], first ? f32x4_t{0.f, 0.f, 0.f, 0.f} : ch[t][mt]);
+          ch[t][mt] = mfma16<XT>(A1, B[mt][1], ch[t][mt]);
+        }
       }
     }
   };
@@ -311,7 +337,14 @@ __global__ __launch_bounds__(GW_THREADS, 2) void k_gemm_wide(ThvmGemvArgs a) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
-  const uint32_t nch = (c1 - c0 + U - 1) / U * U;     // run U at a time (zeros past the slice)
+  auto fold = [&] {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) acc[t][mt] += ch[t][mt];
+  };
+  static_assert(T % U == 0 && T % 2 == 0 && (F == 1 || F == T), "a turn is whole turns of the register sets and LDS buffers, and one chain");
+  const uint32_t nch = (c1 - c0 + T - 1) / T * T;     // run T at a time (zeros past the slice)
   // x and weights are both requested U chunks ahead: a wave's loads return in
   // issue order, so the wait for an x chunk is a wait for every weight load
   // issued before it, and a late x load would drain the weights' window
@@ -326,18 +359,20 @@ __global__ __launch_bounds__(GW_THREADS, 2) void k_gemm_wide(ThvmGemvArgs a) {
     }
     xstore(x0, 0);
   }
-  for (uint32_t c = 0; c < nch; c += U) {
+  for (uint32_t c = 0; c < nch; c += T) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const uint32_t s = s0 + (c + u) * GW_KG;        // the chunk's first step
+    for (int f = 0; f < T; f++) {
+      const int u = f % U;
+      const uint32_t s = s0 + (c + f) * GW_KG;        // the chunk's first step
       meet();
       xstore(xv[(u + 1) % U], (u + 1) & 1);           // the next chunk
       xload(xv[(u + 1) % U], s * 64 + (U + 1) * GW_KC);
       __builtin_amdgcn_sched_barrier(0);
-      compute(u & 1, kg, u);
+      compute(u & 1, kg, u, f == 0);
       wload(u, s + kg + U * GW_KG);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (F > 1) fold();
   }
   if (NM) {
 #pragma unroll
