@@ -70,3 +70,31 @@ def test_gemv_rows_at_the_lds_limit(hip, wdt, xdt, M, K):
     got = y.read(np.float32).reshape(M, N)
     # f32 sums of K products in any order: well inside 2^-24 sqrt(K) of the absolute sum
     assert np.all(np.abs(got - xf @ wf.T) <= 1e-5 * (np.abs(xf) @ np.abs(wf).T))
+
+
+@pytest.mark.parametrize("wdt,xdt,K", [(DT_FP8, DT_BF16, 1024), (DT_F16, DT_F16, 768), (DT_F32, DT_F32, 192), (DT_FP8, DT_BF16, 12288)])
+@pytest.mark.parametrize("N", [2048, 2050, 4096, 4098, 8190, 8192, 16382, 16384])
+def test_gemv_rows_per_wave_keep_the_bits(hip, wdt, xdt, K, N):
+    """One or two weight rows a wave, as the shape picks it on each side of its
+    lines, are the same sums."""
+    print(f"case: gemv rows per wave wdt={wdt} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(N + K)
+    x = rng.standard_normal((4, K)).astype(np.float32)
+    x = x if xdt == DT_F32 else O.encode(x, xdt)
+    wn = {DT_FP8: 1, DT_F16: 2, DT_F32: 4}[wdt]
+    w = O.encode((rng.standard_normal((256, K)) * 0.05).astype(np.float32), wdt) if wdt != DT_F32 else \
+        (rng.standard_normal((256, K)) * 0.05).astype(np.float32)
+    w = np.tile(w, (N // 256 + 1, 1))[:N]
+    assert w.itemsize == wn
+    args = [up(hip, w)] + ([up(hip, rng.random(N).astype(np.float32))] if wdt == DT_FP8 else [])
+    g, b = (up(hip, rng.standard_normal(K).astype(np.float32)) for _ in range(2))
+    for norm in (0, 1, 2) if K <= 8192 else (0,):
+        for M in (1, 2, 3, 4):
+            out = []
+            for kw in ({}, dict(r=1)):
+                y = hip.Buffer(M * N * 4)
+                hip.builtin("gemv", [y, up(hip, x[:M]), *args, *[g, b][:norm]], m=M, n=N, k=K, wt=wdt, xt=xdt, yt=DT_F32,
+                            norm=norm, eps=1e-5, waves=8, **kw)
+                out.append(y.read(np.uint32))
+                y.free()
+            assert np.array_equal(*out), (norm, M)
