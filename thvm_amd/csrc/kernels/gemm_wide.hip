@@ -27,13 +27,18 @@ WIDE_PICKERS(WIDE_DECL)
 //    2048 x 4096    5.6 /  7.2   6.0 /  7.3   7.0 /  7.3  11.4 /  9.6
 //    6400 x 1600    5.3 /  6.8   5.6 /  6.9   6.3 /  6.9   9.2 /  9.4   small: k_gemm
 //    1600 x 1600    4.2 /  6.3   4.3 /  6.5   5.0 /  6.5   7.1 /  8.9
+// and this kernel's time over k_gemm's on the far side of the lines: 4096 x 2048
+// (and 6400, 8192 x 1600) M 33 1.06..1.21, M 48 1.02..1.15, M 64 0.99..1.08; 16-bit
+// 4096, 8192 x 6144 M 17 1.04..1.07 (M 24 1.00).
 // At 16 rows and fewer the widest N gain 4..25% too, and a long K 10% at 16;
 // the line stays at 16 because k_gemm also takes a norm ahead of the product
 // there, and a decoder of 5 to 16 rows holds no workspace.
 extern "C" int thvm_k_gemm_wide_use(const ThvmGemvArgs *a) {
   if (a->seq) return 1;
   if (a->M <= 16) return 0;
-  return a->M > 64 || a->N >= 10240 || a->K >= 6144 || (a->M > 32 && (uint64_t)a->N * a->K >= (8u << 20));
+  if (a->M > 64 || a->N >= 10240) return 1;
+  if (a->K >= 6144) return a->M >= 24 || a->wdt == THVM_DT_FP8E4M3 || a->K >= 8192;
+  return a->M > 32 && a->K >= 2048 && (uint64_t)a->N * a->K >= (a->K >= 4096 ? 8u << 20 : 12u << 20);
 }
 
 // Tile and splits.  One block of 8 waves is resident per CU (more than 128
@@ -41,7 +46,10 @@ extern "C" int thvm_k_gemm_wide_use(const ThvmGemvArgs *a) {
 //   * one tile of x rows (M <= 64; bound by the weight stream): 64 weight rows
 //     per block while that makes at most 256 blocks, else 128, and 256 for the
 //     widest N (an LM head runs many rounds anyway: 128256 x 4096 at M = 60,
-//     113 us with 128 rows, 102 with 256);
+//     113 us with 128 rows, 102 with 256).  Behind a fused norm over more than 32
+//     rows every block norms x again, which fp8 weights do not hide: 128 rows
+//     from 129 such tiles on (16384 x 14336, M = 33: 69 us with 64 rows, 51 with
+//     128, k_gemm 61; 10240 x 4096 23 and 18; 14336 x 2048 14.4 and 14.7);
 //   * several (prompt chunks; bound by the MFMA and LDS pipes): the cheapest of
 //     64, 128, 256 rows by rounds x chunks x the measured time of a chunk
 //     (0.40, 0.56 and 1.04 us), e.g. at M = 299: 6144 x 4096 128 rows 22.4 us
@@ -57,12 +65,14 @@ static void wide_plan(const ThvmGemvArgs *a, int *MT, int *NT, uint32_t *SP) {
   const uint64_t mt = tiles_of(a->M, 16u * *MT), g64 = tiles_of(a->N, 64);
   const uint32_t CH = (a->K / 64 + GW_KG - 1) / GW_KG;
   static const float chunk[3] = {0.40f, 0.56f, 1.04f};
+  const bool xbound = a->norm && a->wdt == THVM_DT_FP8E4M3 && a->M > 32 && a->K >= 4096;
+  const int one = g64 <= (xbound ? 128 : 256) ? 1 : g64 <= 512 ? 2 : 4;
   float best = 0.f;
   *NT = 1;
   *SP = 1;
   for (int i = 0; i < 3; i++) {
     const int nt = 1 << i;
-    if (a->tune_r ? (int)a->tune_r != nt : mt == 1 && nt != (g64 <= 256 ? 1 : g64 <= 512 ? 2 : 4)) continue;
+    if (a->tune_r ? (int)a->tune_r != nt : mt == 1 && nt != one) continue;
     const uint64_t blocks = (g64 + nt - 1) / nt * mt;
     const uint32_t smax = a->tune_blocks ? a->tune_blocks
                         : blocks == 0 || blocks >= 256 ? 1 : 256 / blocks < 8 ? (uint32_t)(256 / blocks) : 8;
