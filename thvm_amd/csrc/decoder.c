@@ -515,12 +515,16 @@ typedef struct { int kind; u32 g, b; } NormSpec;
  * every block takes the rows' statistics (dims it holds in registers), so it is
  * for grids of one round: 256 blocks of 2 16-row tiles (us in a graph, fp16, 8
  * rows, norm and GEMM in two launches -> one: 4800 x 1600 9.4 -> 8.7, 2304 x 768
- * 7.4 -> 6.9; with 4 tiles a block 16384 x 1600 17.2 -> 22.2, from spills). */
+ * 7.4 -> 6.9; with 4 tiles a block 16384 x 1600 17.2 -> 22.2, from spills).  One
+ * launch's time over two, N = 256..8192: dims 768..2048 with 16-bit weights 5
+ * rows 0.86..0.96, 16 rows 0.94..1.06; fp8 0.90..0.95, 12 rows 0.94..1.02, 16 rows
+ * 1.01..1.08; dim 256 8 rows 0.95..1.04, 12 and 16 rows 1.00..1.14. */
 static int fused_norms(const Decoder *d, const NormSpec *ns, u32 n) {
   const char *e = getenv("THVM_HIP_UNFUSED_NORM");
   if (e && e[0] == '1') return 0;
   if (d->rows <= 4 || (ns->kind == 1 && d->c.adtype == THVM_DT_BF16)) return 1;
-  return d->rows <= 16 && d->c.adtype != THVM_DT_FP32 && d->c.dim <= 2048 && n <= 8192 ? 2 : 0;
+  const u32 most = d->c.dim < 768 ? 8 : d->c.wdtype == THVM_DT_FP8E4M3 ? 12 : 16;
+  return d->rows <= most && d->c.adtype != THVM_DT_FP32 && d->c.dim <= 2048 && n <= 8192 ? 2 : 0;
 }
 
 static int emit_norm(Decoder *d, const NormSpec *ns, u32 n, u32 *gin, char *nspec, size_t nlen,
