@@ -265,13 +265,16 @@ extern "C" int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int 
   // at 3; 2304 x 768 with a LayerNorm in pairs, 144 blocks: 6.52 -> 5.64 at 6).
   // Three waves only where they stage x in one pass, four above (256..768 rows
   // of 8192..28672 fp8: 4 waves 0.92..1.01 of the time of 8, 3 waves 0.96..1.03).
+  // 5 to 7 waves without a norm only over rows of 512 chunks and more (1536 rows:
+  // 0.85..1.00 of the time of 8 there, 1.01..1.04 over shorter ones).
   // Not with a fused RMSNorm, whose sum is in the order of a 512-thread block
   // (the persistent step's).
   if (!a->tune_waves && Mk == 1 && chunks == 1 && !xsum && a->norm != 1 && Gr <= 2048) {
     const uint32_t w = (Gr + 255) / 256, wmin = a->norm ? (uint32_t)((a->K + XREG * 64 - 1) / (XREG * 64)) : 1u;
     const uint32_t pass3 = 4u * 64u * 3u * (a->xdt == THVM_DT_FP32 ? 4u : 8u);
     const uint32_t few = a->K <= pass3 ? 3 : 4, lo = wmin > few ? wmin : few;
-    waves = w < lo ? lo : w > 8 ? 8 : w;
+    const bool eight = w > 8 || (w > 4 && !a->norm && (uint64_t)a->K * wsz / 16 < 512);
+    waves = w < lo ? lo : eight ? 8 : w;
   }
   if (Mk > 1 && waves > 8) waves = 8;   // the instances' block limit; the sums do not depend on it
   if (xsum && a->K > 2u * GEMV_SQ * 64u * waves) {   // the staging's element pairs per thread
