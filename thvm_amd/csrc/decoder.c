@@ -6,7 +6,8 @@
  * (bench/dsv2_decode_bench.c: model_init, step_build :2328-2430, capture +
  * replay :2898-3008) and of the GPT-2 driver (bench/gpt2/thvm_gpt2.py:96-131).
  * As there, the token and the position live in device buffers (argmax writes
- * the next token, len_bump advances L), so a replay needs no host values.
+ * the next token and, in a greedy step, advances L; a sampling step ends with
+ * len_bump), so a replay needs no host values.
  *
  * Step (LLAMA, per layer):
  *   norm   xn = rms(x) * g_attn                       -> bf16
@@ -16,7 +17,8 @@
  *   norm   xn = rms(x) * g_ffn
  *   gemv   h = silu(xn Wg^T) * (xn Wu^T)              (rows interleaved g/u)
  *   gemv   x = x + h Wd^T
- * then final norm, LM head (f32 logits), argmax -> tok / history, len_bump.
+ * then final norm, LM head (f32 logits), argmax -> tok / history, L + 1 (when
+ * sampling, the draw and then len_bump).
  * GPT2 swaps RMSNorm for LayerNorm (+bias), RoPE for learned positions,
  * SwiGLU for GELU, and ties the LM head to the token embedding.
  *
@@ -909,7 +911,7 @@ static int build_gpt2(Decoder *d) {
  * per layer [RMSNorm + q|kv GEMV -> mla_prep -> mla_attn (split + merge +
  * W_uv) -> o GEMV + residual -> post-attention RMSNorm -> dense SwiGLU FFN
  * (first_dense layers) or router GEMV + route + expert gate/up + expert down
- * with residual] -> final RMSNorm (f32) -> LM head -> argmax -> len_bump. */
+ * with residual] -> final RMSNorm (f32) -> LM head -> argmax (and L + 1). */
 
 /* YaRN-corrected RoPE tables for the pe dims, [max_seq][d_rope/2]: the
  * DeepSeek-V2-Lite rope scaling (factor 40 over an original 4096-position

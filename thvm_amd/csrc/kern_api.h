@@ -105,8 +105,9 @@ typedef struct ThvmGemvArgs {
 int thvm_k_tile_w(void *y, const void *w, uint32_t N, uint32_t K, uint32_t es, uint32_t lb, hipStream_t s,
                   char *err, int errlen);
 /* y = epi(x . W^T): the GEMV for M <= 4, the MFMA GEMM for M <= 64 (fp16 W
- * with fp16 x, bf16 W with bf16 x, fp8 W with bf16/fp16 x; K % 64 == 0; no
- * fused norm). */
+ * with fp16 x, bf16 W with bf16 x, fp8 W with bf16/fp16 x; K % 64 == 0; norm 1
+ * over bf16 x, or pre), the wide MFMA GEMM with `wide` where
+ * thvm_k_gemm_wide_use says so (M up to 65536). */
 int thvm_k_gemv(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen);
 int thvm_k_gemm_mfma(const ThvmGemvArgs *a, hipStream_t s, char *err, int errlen);
 /* The same for many x rows (above 16; prompt chunks of hundreds): x shared by
