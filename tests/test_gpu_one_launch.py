@@ -11,8 +11,8 @@ from test_gpu_kernels import NP_STORE, SZ, attn_close, rand_store
 
 pytestmark = pytest.mark.gpu
 
-# H, Hkv, hd, chunks, B, cache type: each side of the work and block-count
-# lines, 1 / 8 / 9 / 16 chunks, the three head groups
+# H, Hkv, hd, chunks, B, cache type: each side of the lines in (row, kv head)
+# pairs (96, 192) and chunks (8, 10, 16), the three head groups
 ATTN = [(4, 4, 64, 1, 2, DT_F32), (4, 4, 64, 8, 2, DT_F32), (12, 12, 64, 8, 1, DT_F16), (3, 3, 128, 8, 1, DT_BF16),
         (12, 12, 64, 9, 1, DT_F16), (2, 2, 64, 12, 3, DT_BF16), (2, 2, 64, 13, 3, DT_BF16),
         (4, 4, 64, 9, 1, DT_F32), (26, 26, 64, 16, 5, DT_F16), (16, 16, 64, 16, 8, DT_F32), (16, 16, 128, 9, 8, DT_BF16),

@@ -1,7 +1,8 @@
-"""The GEMV at two to four x rows stages all rows at once and keeps fewer chunks
-in flight than at one: every row must still be the one-row launch's bits, with
-no norm and each fused norm, over row lengths from one vector per thread to the
-most a fused norm takes and weight rows of every chunk remainder."""
+"""The GEMV at two to four x rows stages all rows at once, in an instance per
+fused norm (a LayerNorm's ahead of the weights): every row must still be the
+one-row launch's bits, with no norm and each fused norm, over row lengths from
+one vector per thread to the most a fused norm takes and weight rows of every
+chunk remainder."""
 import numpy as np
 import pytest
 
