@@ -12,14 +12,15 @@ from test_gpu_kernels import NP_STORE, SZ, attn_close, rand_store
 pytestmark = pytest.mark.gpu
 
 # H, Hkv, hd, chunks, B, cache type: each side of the lines in (row, kv head)
-# pairs (96, 192) and chunks (8, 10, 16), the three head groups
+# pairs (96), chunks (8, 16) and a block's work (768, 1536), the three head groups
 ATTN = [(4, 4, 64, 1, 2, DT_F32), (4, 4, 64, 8, 2, DT_F32), (12, 12, 64, 8, 1, DT_F16), (3, 3, 128, 8, 1, DT_BF16),
         (12, 12, 64, 9, 1, DT_F16), (2, 2, 64, 12, 3, DT_BF16), (2, 2, 64, 13, 3, DT_BF16),
         (4, 4, 64, 9, 1, DT_F32), (26, 26, 64, 16, 5, DT_F16), (16, 16, 64, 16, 8, DT_F32), (16, 16, 128, 9, 8, DT_BF16),
         (8, 4, 128, 6, 2, DT_BF16), (8, 4, 128, 7, 2, DT_BF16), (8, 2, 128, 3, 1, DT_BF16), (8, 2, 128, 4, 1, DT_F16),
         (64, 16, 128, 8, 8, DT_BF16), (8, 1, 64, 3, 2, DT_BF16),
         (12, 12, 64, 2, 16, DT_F32), (38, 38, 64, 8, 5, DT_F16), (48, 24, 128, 5, 8, DT_BF16), (64, 16, 64, 3, 12, DT_F16),
-        (12, 12, 64, 11, 8, DT_F16), (19, 19, 128, 9, 5, DT_BF16), (3, 3, 64, 10, 1, DT_F16), (3, 3, 64, 11, 1, DT_F16)]
+        (12, 12, 64, 11, 8, DT_F16), (19, 19, 128, 9, 5, DT_BF16), (3, 3, 64, 10, 1, DT_F16), (3, 3, 64, 11, 1, DT_F16),
+        (76, 19, 128, 8, 5, DT_BF16), (64, 16, 128, 8, 6, DT_BF16), (38, 19, 128, 7, 5, DT_F32), (32, 16, 128, 7, 6, DT_F32)]
 
 
 @pytest.mark.parametrize("H,Hkv,hd,ns,B,cdt", ATTN)

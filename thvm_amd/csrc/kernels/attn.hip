@@ -609,25 +609,34 @@ static bool attn_mf_can(const ThvmAttnArgs *a) {
 // One launch in which a block takes every chunk of its (row, kv head) and
 // writes the output itself, as fused = 2 picks it: no partials, and none of
 // the ~3 us that their hand-off (or a second launch) takes.  What it gives up
-// is the chunks running side by side, so it is for calls whose (row, kv head)
-// pairs fill the chip by themselves.  Measured on gfx950, this form's time over
-// that of the form picked else, in a graph, a full cache / half of one:
-//   2 to 8 chunks, G 1, 2, 4, hd 64 (fp16, f32) and 128 (bf16):
-//     8..64 pairs   1.05..1.97 / 0.93..1.31 (bf16 hd 128 G 1 has faster spots)
-//     96, 128       0.92..1.30 / 0.70..1.07
-//     192..256      0.78..0.99 / 0.62..0.87
-//   9 to 16 chunks, G 1:
-//     8..64 pairs   fp16 hd 64 9 chunks 0.81..0.92 / 0.64..0.71, 12 chunks
-//                   0.96..1.10 / 0.71..0.79, 16 1.10..1.33; others 0.85..1.86
-//     96..256       0.66..1.01 / 0.55..0.89
-//   G 4 (9 to 16 chunks, 16 bits): 1.00..3.47 / 0.91..2.19.
+// is the chunks running side by side, so the line lies at a block's work,
+// n_split G hd products a cache row; with 96 pairs and more the other forms
+// have little left to spread over, and it wins at any work up to 8 chunks.
+// Measured on gfx950 inside decode layers in one graph (a launch timed back to
+// back with itself says otherwise: the split looks better with few pairs), us a
+// layer more (+) or less (-) than the form picked else, over 1 to 256 pairs and
+// hd 64 (fp16, f32) and 128 (bf16), a full cache / half of one:
+//   3 to 8 chunks, against the split's one launch:
+//     below 96 pairs     work <= 768  -2.5..+0.0 / -3.1..-0.7
+//                        1024         -1.6..+0.9 / -1.8..-0.6
+//                        1536         -1.6..+1.7 / -1.9..-1.3
+//                        2048         +0.2..+3.2 / -1.8..-0.1
+//                        4096         +3.8..+5.2 / -0.7..-0.2
+//     96 pairs and more  <= 4096      -7.6..-0.4 / -7.1..-0.6
+//   9 to 16 chunks, against two launches:
+//     G 1, below 96      16 bits, work <= 768  -1.8..+0.7 / -3.1..-1.5
+//                        16 bits, more         -0.2..+6.0 / -2.6..+1.6
+//                        f32                   -1.3..+4.1 / -2.4..-0.1
+//     G 1, 96 and more                         -4.8..+1.3 / -4.5..-2.1
+//     G 2 and 4, below 96                      +0.2..+19.1 / -2.1..+8.5
+//                96 and more                   -3.5..+10.9 / -3.2..+1.7
 // The forced one-launch form (fused = 1) keeps the split of auto_cpb.
 static bool attn_whole(const ThvmAttnArgs *a) {
   const uint32_t G = a->Hkv ? a->H / a->Hkv : 0, bh = a->B * a->Hkv;
   if (a->fused != 2 || a->mf == 1 || (a->cpb && a->cpb < a->n_split) || (G != 1 && G != 2 && G != 4)) return false;
-  if (a->n_split <= 8) return bh >= 192;
-  return G == 1 && a->n_split <= 16 &&
-         (bh >= 96 || (a->cdt != THVM_DT_FP32 && a->hd == 64 && a->n_split <= 10));
+  const uint64_t work = (uint64_t)a->n_split * G * a->hd;
+  if (a->n_split <= 8) return work <= 1536 || bh >= 96;
+  return G == 1 && a->n_split <= 16 && (bh >= 96 || (a->cdt != THVM_DT_FP32 && work <= 768));
 }
 
 // split and merge in one launch: asked for, or the shape's pick
